@@ -2118,15 +2118,13 @@ emel_status gen_execute(const GenReq &q, Route route, int concat_axis, emel_stre
         a.m = q.s0->ne[1];
         a.n = route == Route::MulMatF32 ? q.s1->ne[0] : q.s1->ne[1];
         a.f16 = route == Route::MulMatF16;
-        a.argmax = route == Route::MulMatArgmax;
+        if (route != Route::MulMatArgmax) return launched(emel::launch_generic_mul_mat(a, hs));
         a.index_out = q.r.index_out;
         StreamLease lease;
-        if (a.argmax) {
-            s = lease.acquire(hs);
-            if (s == EMEL_OK) s = lease.work(emel::generic_workspace_bytes(emel::GenWork::MulMatArgmax), &a.workspace);
-            if (s != EMEL_OK) return s;
-        }
-        return launched(emel::launch_generic_mul_mat(a, hs));
+        s = lease.acquire(hs);
+        if (s == EMEL_OK) s = lease.work(emel::generic_workspace_bytes(emel::GenWork::MulMatArgmax), &a.workspace);
+        if (s != EMEL_OK) return s;
+        return launched(emel::launch_generic_mul_mat_argmax(a, hs));
     }
     default:
         return fail(EMEL_ERR_INTERNAL, "unrouted generic request");

@@ -23,8 +23,8 @@
 //                   k_l2_apply over every element;
 //   k_count_*       an exact integer count (count_equal's f32 counter
 //                   saturates at 2^24, which min() reproduces);
-//   k_mm_*          one lane per output element (mul_mat F32 / F16) or per
-//                   row (mul_mat_argmax), the inner products in order.
+//   k_mm_argmax_*   one lane per row (mul_mat_argmax), the inner products in
+//                   order (mul_mat itself: mulmat.hip).
 // Operands are addressed through their own extents and element strides, the
 // reference's coordinates_for_index/byte_offset (generic.rs:896-933), walked
 // incrementally along a row instead of re-decoded per element.
@@ -321,50 +321,6 @@ __global__ __launch_bounds__(kBlock) void k_count_final(const unsigned long long
     }
 }
 
-// ---- mul_mat (generic.rs:1422-1450, :1482-1515) ------------------------------------
-
-// F32: lhs [k, m], rhs [n, k], dst [n, m]; dst(col, row) = sum over inner of
-// lhs(inner, row) * rhs(col, inner), one fused multiply-add per step.
-__global__ __launch_bounds__(kBlock) void k_mm_f32(GenMatArgs a)
-{
-    const float *l = static_cast<const float *>(a.lhs.data);
-    const float *r = static_cast<const float *>(a.rhs.data);
-    float *y = static_cast<float *>(a.y.data);
-    const uint64_t total = a.m * a.n;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; t < total; t += stride) {
-        const uint64_t row = t / a.n;
-        const uint64_t col = t - row * a.n;
-        const float *lp = l + static_cast<int64_t>(row) * a.lhs.st[1];
-        const float *rp = r + static_cast<int64_t>(col) * a.rhs.st[0];
-        float v = 0.0f;
-        for (uint64_t i = 0; i < a.k; ++i)
-            v = __builtin_fmaf(lp[static_cast<int64_t>(i) * a.lhs.st[0]], rp[static_cast<int64_t>(i) * a.rhs.st[1]], v);
-        y[static_cast<int64_t>(col) * a.y.st[0] + static_cast<int64_t>(row) * a.y.st[1]] = v;
-    }
-}
-
-// F16: dense lhs [k, m] and rhs [k, n]; dst [m, n] f32 gets the f64 sum of
-// the f32 products of the widened halves.
-__global__ __launch_bounds__(kBlock) void k_mm_f16(GenMatArgs a)
-{
-    const uint16_t *l = static_cast<const uint16_t *>(a.lhs.data);
-    const uint16_t *r = static_cast<const uint16_t *>(a.rhs.data);
-    float *y = static_cast<float *>(a.y.data);
-    const uint64_t total = a.m * a.n;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; t < total; t += stride) {
-        const uint64_t col = t / a.m;
-        const uint64_t row = t - col * a.m;
-        const uint16_t *lp = l + row * a.k;
-        const uint16_t *rp = r + col * a.k;
-        double s = 0.0;
-        for (uint64_t i = 0; i < a.k; ++i)
-            s += static_cast<double>(emel_fp16_to_f32(lp[i]) * emel_fp16_to_f32(rp[i]));
-        y[static_cast<int64_t>(row) * a.y.st[0] + static_cast<int64_t>(col) * a.y.st[1]] = static_cast<float>(s);
-    }
-}
-
 // mul_mat_argmax: per row of lhs [k, rows] the fused dot with rhs [k], then
 // the first row with the greatest dot.  A sequential scan from row 0 with a
 // strict > keeps row 0 when its dot is NaN; otherwise the result is the
@@ -653,24 +609,16 @@ hipError_t launch_generic_count_equal(const GView &a, const GView &b, float *dst
     return hipGetLastError();
 }
 
-hipError_t launch_generic_mul_mat(const GenMatArgs &a, hipStream_t s)
+hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &a, hipStream_t s)
 {
-    if (a.argmax) {
-        char *ws = static_cast<char *>(a.workspace);
-        float *row0 = reinterpret_cast<float *>(ws);
-        MmBest *partial = reinterpret_cast<MmBest *>(ws + 256);
-        const uint32_t blocks = grid_for(a.m, kBlock, kMmArgmaxBlocks);
-        k_mm_argmax_partial<<<blocks, kBlock, 0, s>>>(a, partial, row0);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        k_mm_argmax_final<<<1, kBlock, 0, s>>>(partial, blocks, row0, static_cast<float *>(a.y.data), a.index_out);
-        return hipGetLastError();
-    }
-    const dim3 grid(grid_for(a.m * a.n, kBlock, 65536));
-    if (a.f16)
-        k_mm_f16<<<grid, kBlock, 0, s>>>(a);
-    else
-        k_mm_f32<<<grid, kBlock, 0, s>>>(a);
+    char *ws = static_cast<char *>(a.workspace);
+    float *row0 = reinterpret_cast<float *>(ws);
+    MmBest *partial = reinterpret_cast<MmBest *>(ws + 256);
+    const uint32_t blocks = grid_for(a.m, kBlock, kMmArgmaxBlocks);
+    k_mm_argmax_partial<<<blocks, kBlock, 0, s>>>(a, partial, row0);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_mm_argmax_final<<<1, kBlock, 0, s>>>(partial, blocks, row0, static_cast<float *>(a.y.data), a.index_out);
     return hipGetLastError();
 }
 

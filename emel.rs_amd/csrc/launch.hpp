@@ -194,12 +194,13 @@ struct GenMatArgs {
     GView lhs, rhs, y;
     uint64_t k, m, n; // argmax: m = rows of lhs
     bool f16;         // dense F16 operands (strides in halves)
-    bool argmax;
-    int32_t *index_out;
-    void *workspace;
+    int32_t *index_out; // argmax only
+    void *workspace;    // argmax only
 };
 
+// mul_mat (mulmat.hip)
 hipError_t launch_generic_mul_mat(const GenMatArgs &args, hipStream_t stream);
+hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &args, hipStream_t stream);
 
 // ---- row gather (getrows.hip) -------------------------------------------------
 

@@ -1,0 +1,475 @@
+// mulmat.hip -- gfx950 kernels for the generic envelope's mul_mat (F32, F16)
+// and mul_mat_argmax (crates/emel-kernels/src/any/generic.rs:1422-1515).
+//
+// The reference adds each output's products in the order of the inner
+// dimension: one fused multiply-add per step in f32 (F32 operands), or an f64
+// sum of f32 products (F16 operands; the product of two halves is exact in
+// f32, so each step is one fused multiply-add in f64).  The matrix
+// instructions v_mfma_f32_16x16x4_f32 and v_mfma_f64_16x16x4_f64 add their
+// four products in that order, each with a single rounding, with denormals,
+// so a chain of them over the inner dimension gives the sequential loop's
+// bits (tests/test_gpu_generic.py compares them with the oracle).  Nothing is
+// split along the inner dimension.
+//
+// Bound by those instructions where the outputs fill the chip (k = m = 4096,
+// n = 512: F16 297 us, 58 TFLOP/s of the 73 that a large f64 product reaches;
+// F32 164 us, 105 of 153) and by the latency of their chains where they do
+// not (n = 1: 23 us, F32 33).  A lane per output that walked both operands in
+// global memory took 32.1 ms for the first.
+//
+//   k_mm_tile   a workgroup per tile of the output, operands staged in LDS
+//   k_mm_any    a lane per output, for strides that a tile's 32-bit offsets
+//               cannot span
+#include <type_traits>
+
+#include "common.hpp"
+#include "launch.hpp"
+#include "libm_replica.hpp"
+
+namespace emel {
+namespace {
+
+typedef float acc4f __attribute__((ext_vector_type(4)));
+typedef double acc4d __attribute__((ext_vector_type(4)));
+
+// One product: y[i * y_si + j * y_sj] = sum over kk of p(i, kk) q(j, kk).
+// j is the output's contiguous dimension in the reference's layouts, so the
+// 16 lanes of a result row store 64 contiguous bytes.  Strides are in
+// elements and not negative.
+struct MmArgs {
+    const void *p; // rows i: element (i, kk) at i * p_si + kk * p_sk
+    const void *q; // element (j, kk) at j * q_sj + kk * q_sk
+    float *y;
+    int64_t p_si, p_sk, q_sj, q_sk, y_si, y_sj;
+    uint32_t ni, nj;
+    uint64_t k;
+    uint32_t ti, tj; // tiles along i and j
+};
+
+// ---- tiles -----------------------------------------------------------------
+// A 256-thread workgroup owns TI x TJ outputs.  Blocks of BK inner elements of
+// its operand rows are staged in LDS, two buffers in turn with one barrier per
+// block, and D blocks are in flight in registers: a tile's chain of matrix
+// instructions runs at their latency, so few waves per SIMD have to cover the
+// memory's latency themselves.
+//
+// An f32 or f64 matrix instruction occupies the SIMD's vector issue on this
+// chip (33 cycles for f32 16x16x4, 65 for f64), and every vector instruction
+// beside it adds its own 4 to 8 cycles.  So the loop holds as few as it can:
+// loads are raw buffer loads from a base that advances in scalar registers
+// (out-of-range lanes read zeros, so rows past the end need no clamp), and
+// F16 is widened to f64 while it is staged, once per workgroup.
+//
+// F16's staged row holds BK doubles in 16-byte slots of two: slot (g, u) has
+// the elements kk = 8 u + g and 8 u + 4 + g, so that lane group g = lane / 16
+// of a matrix instruction feeds two instructions with one 128-bit read.  Eight
+// lanes of such a read are served at a time, four of one group with rows 0-3
+// (mod 8) and four of the next with rows 4-7; the slots' order and the rows'
+// stride (kSlotG, kSlotU, kRow) put them in different banks.  F32 rows are
+// staged as they are (p along kk, q along j) and read 4 bytes a lane.
+//
+// SMALL (F16, TI = TJ = 16): v_mfma_f64_4x4x4 takes 16 rows of q against 4
+// rows of p at a third of the latency; each wave owns 4 rows of p.
+//
+// Past the end of the inner dimension p is padded with -0 and q with +0: each
+// padded product is -0, which leaves every sum as it is, signed zeros
+// included.
+// Two waves per SIMD at least: with at most 256 registers a lane the matrix
+// instructions accumulate in vector registers, without copies to and from the
+// accumulation registers at the loop's ends.
+template <bool F16, bool PVEC, bool QVEC, bool SMALL, int FI, int FJ, int WI, int WJ, int BK, int D>
+__global__ __launch_bounds__(kBlock, 2) void k_mm_tile(MmArgs a)
+{
+    static_assert(D % 2 == 0, "the LDS buffers alternate with the register stages");
+    constexpr int TI = SMALL ? 16 : 16 * FI * WI, TJ = SMALL ? 16 : 16 * FJ * WJ;
+    constexpr int kES = F16 ? 2 : 4;
+    constexpr int kChunk = 16 / kES;                    // elements per 128-bit load
+    constexpr int kChunks = BK / kChunk;                // per row of a block
+    // F16: slot (g, u) of a row is g * kSlotG + u * kSlotU, the row's stride 1
+    // (or 2) slots past a multiple of 8.  SMALL reads four rows of p at a time,
+    // so its p slots keep groups 4 apart (mod 8).
+    constexpr bool kWide = kChunks >= 8;
+    constexpr int kSlotG = kWide ? kChunks : 1, kSlotU = kWide ? 1 : 4;
+    constexpr int kPSlotG = SMALL ? kChunks + 4 : kSlotG;
+    constexpr int kRow = F16 ? (4 * kChunks + (kWide ? 1 : 2)) * 16 : BK * 4 + 16; // bytes per staged row
+    constexpr int kPRow = SMALL ? (4 * kPSlotG + 1) * 16 : kRow;                    // and of p
+    constexpr int kQRow = TJ + (TJ % 32 == 0 ? 16 : 0); // floats per staged row of F32's q (along j)
+    constexpr int kBuf = TI * kPRow + (F16 ? TJ * kRow : BK * kQRow * 4);
+    constexpr int kPLoads = TI * kChunks / kBlock;
+    constexpr int kQLoads = F16 ? TJ * kChunks / kBlock : BK * TJ / 4 / kBlock;
+    static_assert(TI * kChunks % kBlock == 0 && (F16 ? TJ * kChunks : BK * TJ / 4) % kBlock == 0, "whole rounds of loads");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kBuf];
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid % kWave;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    // Neighbouring workgroups share the operand of the dimension with more
+    // tiles, the larger one.
+    uint32_t bi, bj;
+    if (a.ti <= a.tj) {
+        bi = blockIdx.x % a.ti;
+        bj = blockIdx.x / a.ti;
+    } else {
+        bj = blockIdx.x % a.tj;
+        bi = blockIdx.x / a.tj;
+    }
+    const uint32_t i0 = bi * TI, j0 = bj * TJ;
+
+    // The tile's first element of p and q, and the bytes from there to the end
+    // of its last row's last element: nothing past them is read.
+    const char *p0 = static_cast<const char *>(a.p) + static_cast<int64_t>(i0) * a.p_si * kES;
+    const char *q0 = static_cast<const char *>(a.q) + static_cast<int64_t>(j0) * a.q_sj * kES;
+    const int64_t ks = static_cast<int64_t>(a.k);
+    const int64_t p_bytes = (static_cast<int64_t>(min(a.ni - i0, static_cast<uint32_t>(TI)) - 1) * a.p_si + (ks - 1) * a.p_sk + 1) * kES;
+    const int64_t q_bytes = (static_cast<int64_t>(min(a.nj - j0, static_cast<uint32_t>(TJ)) - 1) * a.q_sj + (ks - 1) * a.q_sk + 1) * kES;
+    auto block_rsrc = [&](const char *base, int64_t bytes, int64_t sk, uint64_t k0) {
+        const int64_t at = static_cast<int64_t>(k0) * sk * kES;
+        const int64_t left = bytes - at; // clamped to [0, 2^31 - 1], by its high words: scalar compares are 32 bits wide
+        const int32_t high = static_cast<int32_t>(left >> 31);
+        return buffer_rsrc(base + at, high < 0 ? 0u : high > 0 ? 0x7fffffffu : static_cast<uint32_t>(left));
+    };
+    // 16 bytes of an operand row: chunk `off` apart, element `sk` apart.
+    auto load_chunk = [&](BufRsrc r, uint32_t off, uint32_t sk, bool vec) {
+        if (vec) return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+        uint32_t e[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (F16)
+                e[c] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off + 4 * c, 0, 0)) |
+                       (static_cast<uint32_t>(static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off + 4 * c + 2, 0, 0)))
+                        << 16);
+            else
+                e[c] = __builtin_amdgcn_raw_buffer_load_b32(r, off + c * sk, 0, 0);
+        }
+        return make_uint4(e[0], e[1], e[2], e[3]);
+    };
+    const uint32_t p_sib = static_cast<uint32_t>(a.p_si) * kES, p_skb = static_cast<uint32_t>(a.p_sk) * kES;
+    const uint32_t q_sjb = static_cast<uint32_t>(a.q_sj) * kES, q_skb = static_cast<uint32_t>(a.q_sk) * kES;
+
+    // Thread tid loads chunks tid, tid + 256, ... of the block.
+    uint4 rp[D][kPLoads], rq[D][kQLoads];
+    auto load = [&](int d, uint64_t k0) {
+        const BufRsrc pr = block_rsrc(p0, p_bytes, a.p_sk, k0);
+        const BufRsrc qr = block_rsrc(q0, q_bytes, a.q_sk, k0);
+#pragma unroll
+        for (int l = 0; l < kPLoads; ++l) {
+            const uint32_t c = l * kBlock + tid;
+            rp[d][l] = load_chunk(pr, c / kChunks * p_sib + c % kChunks * kChunk * p_skb, p_skb, PVEC);
+        }
+#pragma unroll
+        for (int l = 0; l < kQLoads; ++l) {
+            const uint32_t c = l * kBlock + tid;
+            if constexpr (F16) {
+                rq[d][l] = load_chunk(qr, c / kChunks * q_sjb + c % kChunks * kChunk * q_skb, q_skb, QVEC);
+            } else if constexpr (QVEC) {
+                rq[d][l] = load_chunk(qr, c / (TJ / 4) * q_skb + c % (TJ / 4) * 16, 4, true);
+            } else { // consecutive lanes take consecutive columns
+                uint32_t e[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t v = (4 * l + w) * kBlock + tid;
+                    e[w] = __builtin_amdgcn_raw_buffer_load_b32(qr, v / TJ * q_skb + v % TJ * q_sjb, 0, 0);
+                }
+                rq[d][l] = make_uint4(e[0], e[1], e[2], e[3]);
+            }
+        }
+    };
+    // Elements of a chunk past the inner dimension's end: k is the chunk's
+    // first.
+    auto pad_chunk = [&](uint4 &w, uint64_t k, uint32_t pad) {
+        uint32_t e[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (F16) {
+                e[c] = k + 2 * c >= a.k ? pad : k + 2 * c + 1 >= a.k ? (e[c] & 0xffffu) | (pad & 0xffff0000u) : e[c];
+            } else {
+                e[c] = k + c >= a.k ? pad : e[c];
+            }
+        }
+        w = make_uint4(e[0], e[1], e[2], e[3]);
+    };
+    // Halves 4 t + g of chunk u, widened, to slot (g, u), place t.
+    auto store_f16 = [&](unsigned char *row, uint32_t u, uint32_t slot_g, const uint4 &w) {
+        double2 *o = reinterpret_cast<double2 *>(row) + u * kSlotU;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t w0 = g < 2 ? w.x : w.y, w1 = g < 2 ? w.z : w.w;
+            const uint16_t h0 = static_cast<uint16_t>(g % 2 ? w0 >> 16 : w0);
+            const uint16_t h1 = static_cast<uint16_t>(g % 2 ? w1 >> 16 : w1);
+            o[g * slot_g] = make_double2(hw_fp16_to_f32(h0), hw_fp16_to_f32(h1));
+        }
+    };
+    auto store = [&](int d, uint64_t k0, unsigned char *buf, bool tail) {
+#pragma unroll
+        for (int l = 0; l < kPLoads; ++l) {
+            const uint32_t c = l * kBlock + tid;
+            if (tail) pad_chunk(rp[d][l], k0 + c % kChunks * kChunk, F16 ? 0x80008000u : 0x80000000u);
+            unsigned char *row = buf + c / kChunks * kPRow;
+            if constexpr (F16) store_f16(row, c % kChunks, kPSlotG, rp[d][l]);
+            else *reinterpret_cast<uint4 *>(row + c % kChunks * 16) = rp[d][l];
+        }
+#pragma unroll
+        for (int l = 0; l < kQLoads; ++l) {
+            const uint32_t c = l * kBlock + tid;
+            if constexpr (F16) {
+                if (tail) pad_chunk(rq[d][l], k0 + c % kChunks * kChunk, 0u);
+                store_f16(buf + TI * kPRow + c / kChunks * kRow, c % kChunks, kSlotG, rq[d][l]);
+            } else {
+                uint32_t *sq = reinterpret_cast<uint32_t *>(buf + TI * kPRow);
+                if constexpr (QVEC) {
+                    const uint32_t kk = c / (TJ / 4);
+                    if (tail && k0 + kk >= a.k) rq[d][l] = make_uint4(0, 0, 0, 0);
+                    *reinterpret_cast<uint4 *>(sq + kk * kQRow + c % (TJ / 4) * 4) = rq[d][l];
+                } else {
+                    const uint32_t e[4] = {rq[d][l].x, rq[d][l].y, rq[d][l].z, rq[d][l].w};
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const uint32_t v = (4 * l + w) * kBlock + tid;
+                        sq[v / TJ * kQRow + v % TJ] = tail && k0 + v / TJ >= a.k ? 0u : e[w];
+                    }
+                }
+            }
+        }
+    };
+
+    using Acc = typename std::conditional<F16, acc4d, acc4f>::type;
+    Acc acc[FI][FJ];
+#pragma unroll
+    for (int x = 0; x < FI; ++x)
+#pragma unroll
+        for (int z = 0; z < FJ; ++z) acc[x][z] = Acc{0, 0, 0, 0};
+    double acc_small = 0.0;
+    const uint32_t g = lane / 16, c16 = lane % 16;
+    const uint32_t wi = wave % WI, wj = wave / WI;
+    const bool multiplies = SMALL ? i0 + 4 * wave < a.ni : WI * WJ == kBlock / kWave || wave < WI * WJ;
+    auto multiply = [&](const unsigned char *buf) {
+        if constexpr (F16) {
+            const uint32_t prow = SMALL ? 4 * wave + lane % 4 : wi * FI * 16 + c16;
+            const uint32_t qrow = SMALL ? c16 : wj * FJ * 16 + c16;
+            const double2 *pb = reinterpret_cast<const double2 *>(buf + prow * kPRow) + g * kPSlotG;
+            const double2 *qb = reinterpret_cast<const double2 *>(buf + TI * kPRow + qrow * kRow) + g * kSlotG;
+#pragma unroll
+            for (int u = 0; u < kChunks; ++u) {
+                double2 fp[FI], fq[FJ];
+#pragma unroll
+                for (int x = 0; x < FI; ++x) fp[x] = pb[u * kSlotU + x * 16 * (kPRow / 16)];
+#pragma unroll
+                for (int z = 0; z < FJ; ++z) fq[z] = qb[u * kSlotU + z * 16 * (kRow / 16)];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    if constexpr (SMALL) {
+                        acc_small = __builtin_amdgcn_mfma_f64_4x4x4f64(s ? fq[0].y : fq[0].x, s ? fp[0].y : fp[0].x,
+                                                                       acc_small, 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int x = 0; x < FI; ++x)
+#pragma unroll
+                            for (int z = 0; z < FJ; ++z)
+                                acc[x][z] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                    s ? fp[x].y : fp[x].x, s ? fq[z].y : fq[z].x, acc[x][z], 0, 0, 0);
+                    }
+                }
+            }
+        } else {
+            const float *pf = reinterpret_cast<const float *>(buf + (wi * FI * 16 + c16) * kRow) + g;
+            const float *qf = reinterpret_cast<const float *>(buf + TI * kPRow) + g * kQRow + wj * FJ * 16 + c16;
+#pragma unroll 8
+            for (int s = 0; s < BK / 4; ++s) {
+                float ep[FI], eq[FJ];
+#pragma unroll
+                for (int x = 0; x < FI; ++x) ep[x] = pf[x * 4 * kRow + s * 4];
+#pragma unroll
+                for (int z = 0; z < FJ; ++z) eq[z] = qf[s * 4 * kQRow + z * 16];
+#pragma unroll
+                for (int x = 0; x < FI; ++x)
+#pragma unroll
+                    for (int z = 0; z < FJ; ++z)
+                        acc[x][z] = __builtin_amdgcn_mfma_f32_16x16x4f32(ep[x], eq[z], acc[x][z], 0, 0, 0);
+            }
+        }
+    };
+
+    // Block b is multiplied from one buffer while the next is staged into the
+    // other, between the same two barriers.  The loop has no exit inside and
+    // every load in it is issued, so the later blocks' loads stay outstanding;
+    // its last blocks, the one past the inner dimension's end among them, come
+    // after it.
+    const uint32_t nb = static_cast<uint32_t>((a.k + BK - 1) / BK);
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, d * BK);
+    if (nb == 1) store(0, 0, lds, true);
+    else store(0, 0, lds, false);
+    load(0, D * BK);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t b = 0;
+    for (; b + D + 1 < nb; b += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            constexpr auto next = [](int x) { return (x + 1) % D; };
+            if (multiplies) multiply(lds + (d % 2) * kBuf);
+            store(next(d), 0, lds + ((d + 1) % 2) * kBuf, false);
+            load(next(d), static_cast<uint64_t>(b + d + 1 + D) * BK);
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0); // the next block's conversions would wait for its loads here
+        }
+    }
+#pragma unroll
+    for (int d = 0; d <= D; ++d) {
+        if (b + d < nb) {
+            if (multiplies) multiply(lds + (d % 2) * kBuf);
+            if (b + d + 1 < nb) {
+                store((d + 1) % D, static_cast<uint64_t>(b + d + 1) * BK, lds + ((d + 1) % 2) * kBuf, true);
+                __syncthreads();
+            }
+        }
+    }
+    if (!multiplies) return;
+    if constexpr (SMALL) { // lane: p row lane % 4, q row 4 (lane / 4 % 4) + g
+        const uint32_t i = i0 + 4 * wave + lane % 4, j = j0 + 4 * (c16 / 4) + g;
+        if (i < a.ni && j < a.nj)
+            a.y[static_cast<int64_t>(i) * a.y_si + static_cast<int64_t>(j) * a.y_sj] = static_cast<float>(acc_small);
+        return;
+    }
+    // Result register r of a lane: row 4 g + r (f32) or 4 r + g (f64), column
+    // lane % 16.
+#pragma unroll
+    for (int x = 0; x < FI; ++x)
+#pragma unroll
+        for (int z = 0; z < FJ; ++z)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t i = i0 + (wi * FI + x) * 16 + (F16 ? 4 * r + g : 4 * g + r);
+                const uint32_t j = j0 + (wj * FJ + z) * 16 + c16;
+                if (i < a.ni && j < a.nj)
+                    a.y[static_cast<int64_t>(i) * a.y_si + static_cast<int64_t>(j) * a.y_sj] =
+                        static_cast<float>(acc[x][z][r]);
+            }
+}
+
+template <bool F16, bool SMALL, int FI, int FJ, int WI, int WJ, int BK, int D>
+void launch_tile(MmArgs a, bool pvec, bool qvec, hipStream_t s)
+{
+    constexpr uint32_t TI = SMALL ? 16 : 16 * FI * WI, TJ = SMALL ? 16 : 16 * FJ * WJ;
+    a.ti = (a.ni + TI - 1) / TI;
+    a.tj = (a.nj + TJ - 1) / TJ;
+    const dim3 grid(a.ti * a.tj);
+    if constexpr (F16) {
+        if (pvec) k_mm_tile<true, true, true, SMALL, FI, FJ, WI, WJ, BK, D><<<grid, kBlock, 0, s>>>(a);
+        else k_mm_tile<true, false, false, SMALL, FI, FJ, WI, WJ, BK, D><<<grid, kBlock, 0, s>>>(a);
+    } else {
+        if (pvec && qvec) k_mm_tile<false, true, true, SMALL, FI, FJ, WI, WJ, BK, D><<<grid, kBlock, 0, s>>>(a);
+        else if (pvec) k_mm_tile<false, true, false, SMALL, FI, FJ, WI, WJ, BK, D><<<grid, kBlock, 0, s>>>(a);
+        else k_mm_tile<false, false, false, SMALL, FI, FJ, WI, WJ, BK, D><<<grid, kBlock, 0, s>>>(a);
+    }
+}
+
+template <bool F16>
+__global__ __launch_bounds__(kBlock) void k_mm_any(MmArgs a)
+{
+    using T = typename std::conditional<F16, uint16_t, float>::type;
+    const uint64_t total = static_cast<uint64_t>(a.ni) * a.nj;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+    for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; t < total; t += stride) {
+        const int64_t i = static_cast<int64_t>(t / a.nj), j = static_cast<int64_t>(t % a.nj);
+        const T *p = static_cast<const T *>(a.p) + i * a.p_si;
+        const T *q = static_cast<const T *>(a.q) + j * a.q_sj;
+        typename std::conditional<F16, double, float>::type v = 0;
+        for (int64_t k = 0; k < static_cast<int64_t>(a.k); ++k) {
+            if constexpr (F16)
+                v += static_cast<double>(hw_fp16_to_f32(p[k * a.p_sk]) * hw_fp16_to_f32(q[k * a.q_sk]));
+            else
+                v = __builtin_fmaf(p[k * a.p_sk], q[k * a.q_sk], v);
+        }
+        a.y[i * a.y_si + j * a.y_sj] = static_cast<float>(v);
+    }
+}
+
+uint64_t tiles(uint64_t ni, uint64_t nj, uint64_t t) { return ((ni + t - 1) / t) * ((nj + t - 1) / t); }
+
+bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+} // namespace
+
+namespace {
+
+// Which tile.  A chain of matrix instructions runs at their latency, so the
+// outputs are spread over the SIMDs before tiles grow: 16x16 up to 512 of
+// them (k = m = 4096, n = 32, F16: 39 us against 53 with 32x32 and 169 with
+// 64x64; F32 35, 39, 103) and where one dimension has at most 16 (n = 16: 27,
+// 54, 170 us), 32x32 above (n = 64: 54 us against 72 and 169), and 64x64,
+// which loads and widens least per product, where its two workgroups per CU
+// fill nine tenths of their last round (n = 512: F16 317 us against 348 with
+// 32x32 and 514 with 16x16; k = 704, m = 10533, n = 283 fill 0.81 of it and
+// take 108 against 96).
+template <bool F16>
+void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
+{
+    // the largest tile's rows and block, in bytes
+    constexpr int64_t es = F16 ? 2 : 4, span = 0x7fffffff / es;
+    if (a.p_si > span / 256 || a.p_sk > span / 256 || a.q_sj > span / 256 || a.q_sk > span / 256) {
+        const uint64_t blocks = (static_cast<uint64_t>(a.ni) * a.nj + kBlock - 1) / kBlock;
+        k_mm_any<F16><<<static_cast<uint32_t>(min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
+        return;
+    }
+    const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 512;
+    if (10 * t64 >= 9 * ((t64 + round - 1) / round * round))
+        launch_tile<F16, false, 2, 2, 2, 2, F16 ? 32 : 64, 2>(a, pvec, qvec, s);
+    else if (min(a.ni, a.nj) > 16 && tiles(a.ni, a.nj, 16) > 512)
+        launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
+    else
+        launch_tile<F16, F16, 1, 1, 1, 1, 128, 4>(a, pvec, qvec, s);
+}
+
+} // namespace
+
+hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
+{
+    MmArgs a{};
+    a.k = g.k;
+    uint64_t ni, nj;
+    bool pvec, qvec;
+    if (g.f16) { // dst [m, n] is contiguous along lhs' rows
+        a.p = g.rhs.data;
+        a.q = g.lhs.data;
+        a.p_si = a.q_sj = static_cast<int64_t>(g.k);
+        a.p_sk = a.q_sk = 1;
+        a.y_si = g.y.st[1];
+        a.y_sj = g.y.st[0];
+        ni = g.n;
+        nj = g.m;
+        pvec = qvec = g.k % 8 == 0 && aligned16(a.p) && aligned16(a.q);
+    } else { // dst [n, m] is contiguous along rhs' columns
+        a.p = g.lhs.data;
+        a.q = g.rhs.data;
+        a.p_si = g.lhs.st[1];
+        a.p_sk = g.lhs.st[0];
+        a.q_sj = g.rhs.st[0];
+        a.q_sk = g.rhs.st[1];
+        a.y_si = g.y.st[1];
+        a.y_sj = g.y.st[0];
+        ni = g.m;
+        nj = g.n;
+        pvec = a.p_sk == 1 && a.p_si % 4 == 0 && g.k % 4 == 0 && aligned16(a.p);
+        qvec = a.q_sj == 1 && a.q_sk % 4 == 0 && nj % 4 == 0 && aligned16(a.q);
+    }
+    // Extents past 32 bits run in slabs.
+    const uint64_t slab = uint64_t{1} << 30;
+    const uint64_t es = g.f16 ? 2 : 4;
+    for (uint64_t i = 0; i < ni; i += slab)
+        for (uint64_t j = 0; j < nj; j += slab) {
+            MmArgs b = a;
+            b.p = static_cast<const char *>(a.p) + i * es * static_cast<uint64_t>(a.p_si);
+            b.q = static_cast<const char *>(a.q) + j * es * static_cast<uint64_t>(a.q_sj);
+            b.y = static_cast<float *>(g.y.data) + static_cast<int64_t>(i) * a.y_si + static_cast<int64_t>(j) * a.y_sj;
+            b.ni = static_cast<uint32_t>(ni - i < slab ? ni - i : slab);
+            b.nj = static_cast<uint32_t>(nj - j < slab ? nj - j : slab);
+            if (g.f16) launch_mm<true>(b, pvec, qvec, s);
+            else launch_mm<false>(b, pvec, qvec, s);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
+}
+
+} // namespace emel

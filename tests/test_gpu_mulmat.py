@@ -1,0 +1,79 @@
+"""GPU parity of mul_mat's tiles (emel_generic_dispatch, MUL_MAT) with the oracle, bit for bit: the matrix
+instructions' chains against the reference's sequential loop, at the edges of the tiles and of the staged blocks,
+for every alignment the loads distinguish."""
+import numpy as np
+import pytest
+
+import emel_hip as eh
+import oracle as orc
+from helpers import Pair, assert_bits_equal, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def mul_mat(gpu, lhs, rhs, dst):
+    want = orc.generic(eh.GenericOp.MUL_MAT, lhs.oview(), rhs.oview(), None, dst.oview(), b"", 0, 0, None)
+    for p in (lhs, rhs, dst):
+        p.to(gpu)
+    req = eh.GenericRequest(eh.GenericOp.MUL_MAT, lhs.pview(), rhs.pview(), None, dst.pview(True))
+    assert want == orc.OK and eh.Kernel().process_event(eh.GenericEvent(req)) == eh.Status.OK, eh.last_error()
+    assert_bits_equal(dst.result(), dst.host, f"lhs {lhs.ne} rhs {rhs.ne}")
+
+
+def values(seed, n, kind):
+    g = rng(seed)
+    x = g.standard_normal(n).astype(np.float32)
+    if kind == "wide":  # exponents far apart: every order of additions gives other bits
+        x = np.ldexp(x, g.integers(-12, 12, n)).astype(np.float32)
+    elif kind == "special":
+        at = g.integers(0, n, max(4, n // 2000))
+        x[at] = np.array([np.inf, np.nan, -0.0, 1e-7], np.float32)[np.arange(at.size) % 4]
+    return x
+
+
+# k m n: one element, tile and block edges of each tile (16, 32, 64 outputs; blocks of 64 to 512), k and n that are
+# not whole vectors, and outputs enough for the largest tiles
+SHAPES = [(1, 1, 1), (8, 16, 16), (520, 17, 16), (511, 15, 300), (96, 4096, 1), (1032, 40, 4), (264, 33, 65),
+          (260, 33, 64), (128, 100, 31), (72, 2049, 1025), (67, 2050, 1023), (64, 2048, 1024)]
+
+
+@pytest.mark.parametrize("kind", ["wide", "special"])
+@pytest.mark.parametrize("k,m,n", SHAPES)
+def test_mul_mat_f16_tiles(gpu, k, m, n, kind):
+    lhs = values(k + m, k * m, kind).astype(np.float16).view(np.uint16)
+    rhs = values(k + n, k * n, kind).astype(np.float16).view(np.uint16)
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [k, n, 1, 1]), Pair(np.zeros(m * n, np.float32), [m, n, 1, 1]))
+
+
+@pytest.mark.parametrize("layout", ["dense", "lhs_columns", "rhs_columns", "padded"])
+@pytest.mark.parametrize("k,m,n", SHAPES)
+def test_mul_mat_f32_tiles(gpu, k, m, n, layout):
+    kind = "special" if layout == "dense" else "wide"
+    lhs, lnb, rhs, rnb = values(k + m, k * m, kind), None, values(k + n, k * n, kind), None
+    if layout == "lhs_columns":  # lhs stored along m
+        lnb = [4 * m, 4, 4 * k * m, 4 * k * m]
+    elif layout == "rhs_columns":  # rhs stored along k
+        rnb = [4 * k, 4, 4 * k * n, 4 * k * n]
+    elif layout == "padded":  # rows of a longer stride, one float off a 16-byte boundary
+        lhs, rhs = values(k + m, (k + 3) * m, kind), values(k + n, (n + 5) * k, kind)
+        lnb, rnb = [4, 4 * (k + 3)] + [4 * (k + 3) * m] * 2, [4, 4 * (n + 5)] + [4 * (n + 5) * k] * 2
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1], lnb), Pair(rhs, [n, k, 1, 1], rnb),
+            Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
+
+
+def test_mul_mat_f32_underflow_keeps_signed_zeros(gpu):
+    # products that round to -0 and sums that end there: the staged blocks' padding must not turn them into +0
+    k, m, n = 5, 20, 18
+    lhs = np.full(k * m, -1e-30, np.float32)
+    lhs[: k * 3] = 1e-30
+    rhs = np.full(n * k, 1e-30, np.float32)
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [n, k, 1, 1]), Pair(np.ones(m * n, np.float32), [n, m, 1, 1]))
+
+
+def test_mul_mat_f32_rows_far_apart(gpu):
+    # rows 32 MiB apart: past the tiles' 32-bit offsets
+    k, m, n, row = 6, 3, 4, (1 << 23) + 4
+    lhs = np.zeros(row * m, np.float32)
+    lhs.reshape(m, row)[:, :k] = values(1, k * m, "wide").reshape(m, k)
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1], [4, 4 * row, 4 * row * m, 4 * row * m]),
+            Pair(values(2, k * n, "wide"), [n, k, 1, 1]), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
