@@ -2122,7 +2122,7 @@ emel_status gen_execute(const GenReq &q, Route route, int concat_axis, emel_stre
         a.index_out = q.r.index_out;
         StreamLease lease;
         s = lease.acquire(hs);
-        if (s == EMEL_OK) s = lease.work(emel::generic_workspace_bytes(emel::GenWork::MulMatArgmax), &a.workspace);
+        if (s == EMEL_OK) s = lease.work(emel::mul_mat_argmax_workspace_bytes(), &a.workspace);
         if (s != EMEL_OK) return s;
         return launched(emel::launch_generic_mul_mat_argmax(a, hs));
     }

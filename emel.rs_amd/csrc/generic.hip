@@ -23,8 +23,6 @@
 //                   k_l2_apply over every element;
 //   k_count_*       an exact integer count (count_equal's f32 counter
 //                   saturates at 2^24, which min() reproduces);
-//   k_mm_argmax_*   one lane per row (mul_mat_argmax), the inner products in
-//                   order (mul_mat itself: mulmat.hip).
 // Operands are addressed through their own extents and element strides, the
 // reference's coordinates_for_index/byte_offset (generic.rs:896-933), walked
 // incrementally along a row instead of re-decoded per element.
@@ -321,82 +319,6 @@ __global__ __launch_bounds__(kBlock) void k_count_final(const unsigned long long
     }
 }
 
-// mul_mat_argmax: per row of lhs [k, rows] the fused dot with rhs [k], then
-// the first row with the greatest dot.  A sequential scan from row 0 with a
-// strict > keeps row 0 when its dot is NaN; otherwise the result is the
-// lowest row holding the maximum of the non-NaN dots.
-struct MmBest {
-    float v;
-    uint32_t has;
-    uint64_t i;
-};
-
-__device__ __forceinline__ void mm_merge(MmBest &a, const MmBest &b)
-{
-    if (!b.has) return;
-    if (!a.has || b.v > a.v || (b.v == a.v && b.i < a.i)) a = b;
-}
-
-__global__ __launch_bounds__(kBlock) void k_mm_argmax_partial(GenMatArgs a, MmBest *partial, float *row0)
-{
-    __shared__ MmBest part[kBlock / kWave];
-    const float *l = static_cast<const float *>(a.lhs.data);
-    const float *r = static_cast<const float *>(a.rhs.data);
-    MmBest best{0.0f, 0u, 0ull};
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t row = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; row < a.m; row += stride) {
-        const float *lp = l + static_cast<int64_t>(row) * a.lhs.st[1];
-        float v = 0.0f;
-        for (uint64_t i = 0; i < a.k; ++i)
-            v = __builtin_fmaf(lp[static_cast<int64_t>(i) * a.lhs.st[0]], r[static_cast<int64_t>(i) * a.rhs.st[0]], v);
-        if (row == 0) row0[0] = v;
-        if (v == v) mm_merge(best, MmBest{v, 1u, row});
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        MmBest o;
-        o.v = __shfl_xor(best.v, off, kWave);
-        o.has = __shfl_xor(best.has, off, kWave);
-        o.i = __shfl_xor(best.i, off, kWave);
-        mm_merge(best, o);
-    }
-    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < kBlock / kWave; ++i) mm_merge(best, part[i]);
-        partial[blockIdx.x] = best;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_mm_argmax_final(const MmBest *partial, uint32_t n, const float *row0,
-                                                            float *dst, int32_t *index_out)
-{
-    __shared__ MmBest part[kBlock / kWave];
-    MmBest best{0.0f, 0u, 0ull};
-    for (uint32_t i = threadIdx.x; i < n; i += kBlock) mm_merge(best, partial[i]);
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        MmBest o;
-        o.v = __shfl_xor(best.v, off, kWave);
-        o.has = __shfl_xor(best.has, off, kWave);
-        o.i = __shfl_xor(best.i, off, kWave);
-        mm_merge(best, o);
-    }
-    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < kBlock / kWave; ++i) mm_merge(best, part[i]);
-        const float v0 = row0[0];
-        if (v0 != v0 || !best.has) {
-            dst[0] = v0;
-            index_out[0] = 0;
-        } else {
-            dst[0] = best.v;
-            index_out[0] = static_cast<int32_t>(best.i);
-        }
-    }
-}
-
 uint32_t grid_for(uint64_t count, uint32_t block, uint64_t cap)
 {
     uint64_t blocks = (count + block - 1) / block;
@@ -404,8 +326,6 @@ uint32_t grid_for(uint64_t count, uint32_t block, uint64_t cap)
     if (blocks == 0) blocks = 1;
     return static_cast<uint32_t>(blocks);
 }
-
-constexpr uint32_t kMmArgmaxBlocks = 2048;
 
 } // namespace
 
@@ -563,7 +483,6 @@ uint64_t generic_workspace_bytes(GenWork w)
     switch (w) {
     case GenWork::L2Norm: return 256;
     case GenWork::CountEqual: return kCountBlocks * sizeof(unsigned long long);
-    case GenWork::MulMatArgmax: return 256 + kMmArgmaxBlocks * sizeof(MmBest);
     }
     return 0;
 }
@@ -606,19 +525,6 @@ hipError_t launch_generic_count_equal(const GView &a, const GView &b, float *dst
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     k_count_final<<<1, kBlock, 0, s>>>(partial, blocks, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &a, hipStream_t s)
-{
-    char *ws = static_cast<char *>(a.workspace);
-    float *row0 = reinterpret_cast<float *>(ws);
-    MmBest *partial = reinterpret_cast<MmBest *>(ws + 256);
-    const uint32_t blocks = grid_for(a.m, kBlock, kMmArgmaxBlocks);
-    k_mm_argmax_partial<<<blocks, kBlock, 0, s>>>(a, partial, row0);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    k_mm_argmax_final<<<1, kBlock, 0, s>>>(partial, blocks, row0, static_cast<float *>(a.y.data), a.index_out);
     return hipGetLastError();
 }
 

@@ -179,7 +179,7 @@ struct GenOrdArgs {
 
 hipError_t launch_generic_ordinal(const GenOrdArgs &args, hipStream_t stream);
 
-enum class GenWork : uint32_t { L2Norm = 0, CountEqual, MulMatArgmax };
+enum class GenWork : uint32_t { L2Norm = 0, CountEqual };
 uint64_t generic_workspace_bytes(GenWork which);
 
 hipError_t launch_generic_l2_norm(const GView &x, const GView &y, void *workspace, hipStream_t stream);
@@ -198,8 +198,9 @@ struct GenMatArgs {
     void *workspace;    // argmax only
 };
 
-// mul_mat (mulmat.hip)
+// mul_mat and mul_mat_argmax (mulmat.hip)
 hipError_t launch_generic_mul_mat(const GenMatArgs &args, hipStream_t stream);
+uint64_t mul_mat_argmax_workspace_bytes();
 hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &args, hipStream_t stream);
 
 // ---- row gather (getrows.hip) -------------------------------------------------

@@ -20,6 +20,11 @@
 //   k_mm_tile   a workgroup per tile of the output, operands staged in LDS
 //   k_mm_any    a lane per output, for strides that a tile's 32-bit offsets
 //               cannot span
+//   k_mm_rows   a lane per row of lhs for one column, rows streamed through
+//               LDS: mul_mat with n = 1 and mul_mat_argmax
+//   k_mm_argmax_walk, k_mm_argmax_final
+//               mul_mat_argmax for other layouts, and its merge
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -385,6 +390,211 @@ __global__ __launch_bounds__(kBlock) void k_mm_any(MmArgs a)
     }
 }
 
+// ---- rows ------------------------------------------------------------------
+// One wave takes R rows of lhs against one vector, a lane per row and an fma
+// per element in order.  A lane that walked its own row would touch a cache
+// line per element and wave; here a tile of R x (2048 / R) floats (8 KB) is
+// loaded in full lines, 128 bytes of a row or more at a time, two tiles ahead
+// in registers, and turned in LDS (rows 16 bytes longer than a multiple of
+// 128, so that neither side collides in banks).  The vector's elements are
+// scalar loads.  Bound by memory where the rows fill the chip: the argmax over
+// 151936 rows of 4096 takes 425 us, 5.9 TB/s (3.37 ms with a lane per row in
+// global memory).
+//
+// mul_mat_argmax: the first row with the greatest dot.  A sequential scan from
+// row 0 with a strict > keeps row 0 when its dot is NaN; otherwise the result
+// is the lowest row holding the maximum of the non-NaN dots.  A candidate's
+// key orders by value (-0 as +0), then by lower row; 0 is no candidate.
+struct MmBest {
+    uint64_t key;
+    float v;
+    uint32_t pad;
+};
+
+__device__ __forceinline__ uint64_t mm_key(float v, uint32_t row)
+{
+    if (v != v) return 0;
+    const uint32_t b = __builtin_bit_cast(uint32_t, v + 0.0f);
+    const uint32_t o = b & 0x80000000u ? ~b : b | 0x80000000u;
+    return (static_cast<uint64_t>(o) << 32) | (0xffffffffu - row);
+}
+
+// The wave's greatest key, with its value, in lane 0's result.
+__device__ __forceinline__ MmBest mm_wave_best(MmBest b)
+{
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        const uint64_t k = __shfl_xor(b.key, off, kWave);
+        const float v = __shfl_xor(b.v, off, kWave);
+        if (k > b.key) {
+            b.key = k;
+            b.v = v;
+        }
+    }
+    return b;
+}
+
+template <int R, bool ARGMAX>
+__global__ __launch_bounds__(kWave) void k_mm_rows(const float *__restrict__ l, int64_t st, const float *__restrict__ h,
+                                                   uint64_t k, uint32_t m, float *y, int64_t y_st, MmBest *partial,
+                                                   float *row0)
+{
+    constexpr int D = 2, kTile = 2048 / R, kC = kTile / 4, kRow = kTile * 4 + 16;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[R * kRow];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t nb = static_cast<uint32_t>((k + kTile - 1) / kTile);
+    MmBest best{0, 0.0f, 0};
+    for (uint32_t r0 = blockIdx.x * R; r0 < m; r0 += gridDim.x * R) { // m < 2^31
+        const char *base = reinterpret_cast<const char *>(l + static_cast<int64_t>(r0) * st);
+        const uint32_t rows = m - r0 < R ? m - r0 : R;
+        const int64_t bytes = (static_cast<int64_t>(rows - 1) * st + static_cast<int64_t>(k)) * 4;
+        float4 rv[D][8];
+        auto load = [&](int d, uint32_t b) {
+            const int64_t at = static_cast<int64_t>(b) * (kTile * 4);
+            const int64_t left = bytes - at;
+            const int32_t high = static_cast<int32_t>(left >> 31);
+            const BufRsrc r = buffer_rsrc(base + at, high < 0 ? 0u : high > 0 ? 0x7fffffffu : static_cast<uint32_t>(left));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t c = j * kWave + lane;
+                rv[d][j] = ld_buf_nt(r, c / kC * (static_cast<uint32_t>(st) * 4) + c % kC * 16);
+            }
+        };
+        auto store = [&](int d) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t c = j * kWave + lane;
+                *reinterpret_cast<float4 *>(lds + c / kC * kRow + c % kC * 16) = rv[d][j];
+            }
+        };
+        const float4 *mine = reinterpret_cast<const float4 *>(lds + lane % R * kRow);
+        float v = 0.0f;
+        auto add = [&](const float *hb, int c) {
+            const float4 q = mine[c];
+            v = __builtin_fmaf(q.x, hb[4 * c], v);
+            v = __builtin_fmaf(q.y, hb[4 * c + 1], v);
+            v = __builtin_fmaf(q.z, hb[4 * c + 2], v);
+            v = __builtin_fmaf(q.w, hb[4 * c + 3], v);
+        };
+#pragma unroll
+        for (int d = 0; d < D; ++d) load(d, d);
+        uint32_t b = 0;
+        for (; b + D < nb; b += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                store(d);
+                load(d, b + d + D);
+                __syncthreads();
+                const float *hb = h + static_cast<uint64_t>(b + d) * kTile;
+#pragma unroll
+                for (int c = 0; c < kC; ++c) add(hb, c);
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (b + d < nb) {
+                store(d);
+                __syncthreads();
+                const uint64_t k0 = static_cast<uint64_t>(b + d) * kTile;
+                const int n = static_cast<int>(min<uint64_t>(kTile, k - k0) / 4);
+                for (int c = 0; c < n; ++c) add(h + k0, c);
+                __syncthreads();
+            }
+        }
+        const uint32_t row = r0 + lane;
+        if (lane < rows) {
+            if constexpr (ARGMAX) {
+                if (row == 0) row0[0] = v;
+                const uint64_t key = mm_key(v, row);
+                if (key > best.key) best = MmBest{key, v, 0};
+            } else {
+                y[static_cast<int64_t>(row) * y_st] = v;
+            }
+        }
+    }
+    if constexpr (ARGMAX) {
+        best = mm_wave_best(best);
+        if (lane == 0) partial[blockIdx.x] = best;
+    }
+}
+
+// Other layouts: each lane walks its own row.
+__global__ __launch_bounds__(kBlock) void k_mm_argmax_walk(GenMatArgs a, MmBest *partial, float *row0)
+{
+    const float *l = static_cast<const float *>(a.lhs.data);
+    const float *r = static_cast<const float *>(a.rhs.data);
+    MmBest best{0, 0.0f, 0};
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+    for (uint64_t row = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; row < a.m; row += stride) {
+        const float *lp = l + static_cast<int64_t>(row) * a.lhs.st[1];
+        float v = 0.0f;
+        for (uint64_t i = 0; i < a.k; ++i)
+            v = __builtin_fmaf(lp[static_cast<int64_t>(i) * a.lhs.st[0]], r[static_cast<int64_t>(i) * a.rhs.st[0]], v);
+        if (row == 0) row0[0] = v;
+        const uint64_t key = mm_key(v, static_cast<uint32_t>(row));
+        if (key > best.key) best = MmBest{key, v, 0};
+    }
+    best = mm_wave_best(best);
+    if (threadIdx.x % kWave == 0) partial[blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave] = best;
+}
+
+constexpr int kFinalBlock = 1024;
+
+__global__ __launch_bounds__(kFinalBlock) void k_mm_argmax_final(const MmBest *partial, uint32_t n, const float *row0,
+                                                                 float *dst, int32_t *index_out)
+{
+    __shared__ MmBest part[kFinalBlock / kWave];
+    MmBest best{0, 0.0f, 0};
+    for (uint32_t i = threadIdx.x; i < n; i += kFinalBlock) {
+        const MmBest o = partial[i];
+        if (o.key > best.key) best = o;
+    }
+    best = mm_wave_best(best);
+    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kFinalBlock / kWave; ++i)
+            if (part[i].key > best.key) best = part[i];
+        const float v0 = row0[0];
+        if (v0 != v0 || best.key == 0) {
+            dst[0] = v0;
+            index_out[0] = 0;
+        } else {
+            dst[0] = best.v;
+            index_out[0] = static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(best.key));
+        }
+    }
+}
+
+constexpr uint32_t kMmPartials = 8192; // partial results of one argmax at most
+
+bool rows_vectorisable(const GView &lhs, uint64_t k, const void *h, int64_t h_st)
+{
+    // whole aligned chunks of a row, 64 rows within a buffer's 32-bit offsets
+    return lhs.st[0] == 1 && lhs.st[1] % 4 == 0 && lhs.st[1] < (int64_t{1} << 22) && k % 4 == 0 && (k == 1 || h_st == 1) &&
+           (reinterpret_cast<uintptr_t>(lhs.data) & 15u) == 0 && (reinterpret_cast<uintptr_t>(h) & 3u) == 0;
+}
+
+template <bool ARGMAX>
+uint32_t launch_rows_dot(const GenMatArgs &a, MmBest *partial, float *row0, hipStream_t s)
+{
+    const float *l = static_cast<const float *>(a.lhs.data), *h = static_cast<const float *>(a.rhs.data);
+    float *y = static_cast<float *>(a.y.data);
+    const uint32_t m = static_cast<uint32_t>(a.m);
+    auto go = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((a.m + R - 1) / R, kMmPartials));
+        k_mm_rows<R, ARGMAX><<<blocks, kWave, 0, s>>>(l, a.lhs.st[1], h, a.k, m, y, a.y.st[1], partial, row0);
+        return blocks;
+    };
+    // about 2048 waves or more: 8 per CU, with 16 KB of loads each, cover the
+    // memory's latency (60000 rows of 2048: 84 us, 5.8 TB/s)
+    if (a.m >= 64 * 2048) return go(std::integral_constant<int, 64>{});
+    if (a.m >= 32 * 2048) return go(std::integral_constant<int, 32>{});
+    return go(std::integral_constant<int, 16>{});
+}
+
 uint64_t tiles(uint64_t ni, uint64_t nj, uint64_t t) { return ((ni + t - 1) / t) * ((nj + t - 1) / t); }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -409,13 +619,13 @@ void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
     constexpr int64_t es = F16 ? 2 : 4, span = 0x7fffffff / es;
     if (a.p_si > span / 256 || a.p_sk > span / 256 || a.q_sj > span / 256 || a.q_sk > span / 256) {
         const uint64_t blocks = (static_cast<uint64_t>(a.ni) * a.nj + kBlock - 1) / kBlock;
-        k_mm_any<F16><<<static_cast<uint32_t>(min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
+        k_mm_any<F16><<<static_cast<uint32_t>(std::min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
         return;
     }
     const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 512;
     if (10 * t64 >= 9 * ((t64 + round - 1) / round * round))
         launch_tile<F16, false, 2, 2, 2, 2, F16 ? 32 : 64, 2>(a, pvec, qvec, s);
-    else if (min(a.ni, a.nj) > 16 && tiles(a.ni, a.nj, 16) > 512)
+    else if (std::min(a.ni, a.nj) > 16 && tiles(a.ni, a.nj, 16) > 512)
         launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
     else
         launch_tile<F16, F16, 1, 1, 1, 1, 128, 4>(a, pvec, qvec, s);
@@ -429,6 +639,12 @@ hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
     a.k = g.k;
     uint64_t ni, nj;
     bool pvec, qvec;
+    // One column: the rows' waves need to fill the chip (k = 4096, us with rows
+    // / with tiles: m = 4096 52 / 41, 11008 62 / 50, 16384 56 / 69, 32000 91 / 198).
+    if (!g.f16 && g.n == 1 && g.m >= 16384 && g.m <= 0x7fffffffull && rows_vectorisable(g.lhs, g.k, g.rhs.data, g.rhs.st[1])) {
+        launch_rows_dot<false>(g, nullptr, nullptr, s);
+        return hipGetLastError();
+    }
     if (g.f16) { // dst [m, n] is contiguous along lhs' rows
         a.p = g.rhs.data;
         a.q = g.lhs.data;
@@ -470,6 +686,27 @@ hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
             if (e != hipSuccess) return e;
         }
     return hipSuccess;
+}
+
+uint64_t mul_mat_argmax_workspace_bytes() { return 256 + kMmPartials * sizeof(MmBest); }
+
+hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &a, hipStream_t s)
+{
+    char *ws = static_cast<char *>(a.workspace);
+    float *row0 = reinterpret_cast<float *>(ws);
+    MmBest *partial = reinterpret_cast<MmBest *>(ws + 256);
+    uint32_t n;
+    if (rows_vectorisable(a.lhs, a.k, a.rhs.data, a.rhs.st[0])) {
+        n = launch_rows_dot<true>(a, partial, row0, s);
+    } else {
+        const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((a.m + kBlock - 1) / kBlock, kMmPartials / (kBlock / kWave)));
+        k_mm_argmax_walk<<<blocks, kBlock, 0, s>>>(a, partial, row0);
+        n = blocks * (kBlock / kWave);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_mm_argmax_final<<<1, kFinalBlock, 0, s>>>(partial, n, row0, static_cast<float *>(a.y.data), a.index_out);
+    return hipGetLastError();
 }
 
 } // namespace emel

@@ -77,3 +77,44 @@ def test_mul_mat_f32_rows_far_apart(gpu):
     lhs.reshape(m, row)[:, :k] = values(1, k * m, "wide").reshape(m, k)
     mul_mat(gpu, Pair(lhs, [k, m, 1, 1], [4, 4 * row, 4 * row * m, 4 * row * m]),
             Pair(values(2, k * n, "wide"), [n, k, 1, 1]), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
+
+
+def argmax(gpu, lhs, rhs):
+    dst, idx = Pair(np.zeros(1, np.float32), [1, 1, 1, 1]).to(gpu), np.full(1, -7, np.int32)
+    want = orc.generic(eh.GenericOp.MUL_MAT_ARGMAX, lhs.oview(), rhs.oview(), None, dst.oview(), b"", 0, 0, idx)
+    index = Pair(np.full(1, -7, np.int32), [1, 1, 1, 1]).to(gpu)
+    req = eh.GenericRequest(eh.GenericOp.MUL_MAT_ARGMAX, lhs.to(gpu).pview(), rhs.to(gpu).pview(), None,
+                            dst.pview(True)).with_index_out(index.dev)
+    assert want == orc.OK and eh.Kernel().process_event(eh.GenericEvent(req)) == eh.Status.OK, eh.last_error()
+    assert_bits_equal(dst.result(), dst.host, "value")
+    assert int(index.dev.cpu()[0]) == int(idx[0])
+
+
+# k m: row tails and tile tails of each row count per wave (16, 32, 64 rows; tiles of 128, 64, 32 columns), more row
+# blocks than workgroups, and rows that are not whole vectors
+@pytest.mark.parametrize("k,m", [(4, 1), (132, 15), (260, 33), (512, 17), (68, 65600), (36, 131137), (8, 600001), (37, 50)])
+@pytest.mark.parametrize("case", ["plain", "tie", "zeros", "nan", "nan_first", "all_nan"])
+def test_mul_mat_argmax_rows(gpu, k, m, case):
+    w, h = values(k * m, k * m, "wide"), values(k, k, "wide")
+    rows = w.reshape(m, k)
+    if case == "tie":  # the greatest row, again later
+        rows[m // 2] = np.abs(w).max() * np.sign(h)
+        rows[m - 1] = rows[m // 2]
+    elif case == "zeros":  # every dot +0 or -0: the first row wins with its own sign
+        rows[:] = np.where(np.arange(m) % 2 == 0, np.float32(-1e-30), np.float32(1e-30))[:, None]
+        h[:] = np.float32(1e-30)
+    elif case == "nan":
+        rows[m - 1, k // 2] = np.nan
+    elif case == "nan_first":
+        rows[0, 0] = np.nan
+    elif case == "all_nan":
+        h[0] = np.nan
+    argmax(gpu, Pair(w, [k, m, 1, 1]), Pair(h, [k, 1, 1, 1]))
+
+
+@pytest.mark.parametrize("k,m", [(4, 1), (260, 33), (132, 4097), (36, 131137)])
+def test_mul_mat_f32_one_column(gpu, k, m):
+    # rhs and dst columns apart, lhs rows padded
+    lhs, rhs = values(k + m, (k + 8) * m, "special"), values(k, k, "wide")
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1], [4, 4 * (k + 8)] + [4 * (k + 8) * m] * 2), Pair(rhs, [1, k, 1, 1]),
+            Pair(np.zeros(3 * m, np.float32), [1, m, 1, 1], [4, 12, 12 * m, 12 * m]))
