@@ -6,10 +6,12 @@
 // depends on the order of its additions, so each kernel but k_gen_norm
 // gives one lane the reference's whole loop for its unit of independent
 // work, in the reference's order:
-//   k_gen_rows      one lane per row: cumsum, soft_max_back, rms_norm_back,
-//                   and norm / rms_norm rows narrower than a wave (soft_max
-//                   uses the typed strided path's exact sequential-sum
-//                   kernel);
+//   k_gen_rows      one lane per row: cumsum, soft_max_back and rms_norm_back
+//                   of strided operands, and norm / rms_norm rows narrower
+//                   than a wave (soft_max uses the typed strided path's exact
+//                   sequential-sum kernel);
+//   k_back_rows     soft_max_back and rms_norm_back of dense operands: the
+//                   sums as chains in order, the rest by whole workgroups;
 //   k_gen_norm      a workgroup per row for norm and rms_norm rows of 64 or
 //                   more columns that the typed row kernels cannot take
 //                   (those run vectorisable rows with the generic arithmetic);
@@ -176,6 +178,241 @@ __global__ __launch_bounds__(kRowBlock) void k_gen_rows(GenRowArgs a)
             xi.next(a.x);
             gi.next(a.g);
             yi.next(a.y);
+        }
+    }
+}
+
+// ---- soft_max_back and rms_norm_back over dense operands ---------------------------
+// generic.rs:1849-1926: a row's sums are sequential (one f32 fma chain, or two
+// f64 sums of f32 products), so their order cannot be split; what can be is
+// everything around them.  A workgroup takes `group` whole rows, up to
+// kBackTile elements (wider rows pass in tiles): all its threads load x and g
+// once, 16 bytes a lane, keep them in registers for the result, and stage the
+// chains' operands in LDS; then the chains run side by side:
+//   soft_max_back  a lane per row, x and g from LDS, 7.5 cycles an element;
+//   rms_norm_back  x*x and g*x rounded to f32 by all threads, then added by
+//                  v_mfma_f64_4x4x4 against ones: four sequential f64
+//                  additions of sixteen sums in 22 cycles (a lane that
+//                  converted and added took 16 an element).
+// Bound by those chains for few wide rows (rms_norm_back, 512 rows of 4096:
+// 27 us, of which 13 are the chain; 2027 us with a lane per row walking global
+// memory) and by memory for many (soft_max_back, 16384 rows of 512: 24 us,
+// 4.2 TB/s; 192 us).
+constexpr int kBackVec = 8;                             // float4 of x and of g per thread
+constexpr uint32_t kBackTile = kBackVec * 4 * kBlock;   // elements per workgroup and pass
+constexpr uint32_t kBackRows = 64;                      // rows per workgroup at most (32 for rms_norm_back)
+
+struct BackArgs {
+    const float *x, *g;
+    float *y; // may be x or g
+    uint64_t rows, width;
+    uint32_t group; // rows per workgroup; 1 when width > kBackTile
+    uint32_t ld;    // floats per staged row
+    FastDiv by_width; // of the tile's element index (group > 1)
+    float eps;
+};
+
+// VEC: 16-byte accesses; FOURS: a thread's four elements share a row.
+template <bool RMS, bool VEC, bool FOURS>
+__global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) float s_rows[];
+    __shared__ double s_sum[kBackRows];
+    __shared__ double s_inv[kBackRows];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * a.group;
+    const uint32_t rows = static_cast<uint32_t>(a.rows - r0 < a.group ? a.rows - r0 : a.group);
+    const uint64_t first = r0 * a.width;
+    const double wd = static_cast<double>(a.width);
+    const uint64_t tiles = a.group > 1 ? 1 : (a.width + kBackTile - 1) / kBackTile;
+    float *const s_p = s_rows;
+    float *const s_q = s_rows + a.group * a.ld;
+
+    float4 xv[kBackVec], gv[kBackVec];
+    auto index = [&](int j) { return VEC ? (j * kBlock + tid) * 4 : j * kBlock * 4 + tid; };
+    // element e of slot j: VEC takes four in a row, else every 256th
+    auto elem = [&](int j, int e) { return VEC ? index(j) + e : index(j) + e * kBlock; };
+    // Elements past the tile's n read zeros, and stores there are dropped.
+    auto load = [&](uint64_t at, uint32_t n) {
+        const BufRsrc xr = buffer_rsrc(a.x + at, n * 4), gr = buffer_rsrc(a.g + at, n * 4);
+#pragma unroll
+        for (int j = 0; j < kBackVec; ++j) {
+            if constexpr (VEC) {
+                xv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, index(j) * 4, 0, 0));
+                gv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(gr, index(j) * 4, 0, 0));
+            } else {
+                float xe[4], ge[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    xe[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, elem(j, e) * 4, 0, 0));
+                    ge[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gr, elem(j, e) * 4, 0, 0));
+                }
+                xv[j] = make_float4(xe[0], xe[1], xe[2], xe[3]);
+                gv[j] = make_float4(ge[0], ge[1], ge[2], ge[3]);
+            }
+        }
+    };
+    auto place = [&](uint32_t i) { // the element's place in a staged array
+        const uint32_t r = a.group > 1 ? a.by_width.div(i) : 0;
+        return a.group > 1 ? r * a.ld + (i - r * static_cast<uint32_t>(a.width)) : i;
+    };
+    auto stage = [&](uint32_t n) {
+#pragma unroll
+        for (int j = 0; j < kBackVec; ++j) {
+            float4 p = xv[j], q = gv[j];
+            if constexpr (RMS) {
+                q = make_float4(gv[j].x * xv[j].x, gv[j].y * xv[j].y, gv[j].z * xv[j].z, gv[j].w * xv[j].w);
+                p = make_float4(xv[j].x * xv[j].x, xv[j].y * xv[j].y, xv[j].z * xv[j].z, xv[j].w * xv[j].w);
+            }
+            if constexpr (FOURS) {
+                if (index(j) < n) {
+                    const uint32_t o = place(index(j));
+                    *reinterpret_cast<float4 *>(s_p + o) = p;
+                    *reinterpret_cast<float4 *>(s_q + o) = q;
+                }
+            } else {
+                const float pe[4] = {p.x, p.y, p.z, p.w}, qe[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t i = elem(j, e);
+                    if (i < n) {
+                        const uint32_t o = place(i);
+                        s_p[o] = pe[e];
+                        s_q[o] = qe[e];
+                    }
+                }
+            }
+        }
+    };
+
+    float dot = 0.0f;  // soft_max_back: lane r of wave 0 holds row r's
+    double sums = 0.0; // rms_norm_back: the matrix result, below
+    const uint32_t g4 = lane / 16;
+    for (uint64_t t = 0; t < tiles; ++t) {
+        const uint64_t left = static_cast<uint64_t>(rows) * a.width - t * kBackTile;
+        const uint32_t n = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(left < kBackTile ? left : kBackTile));
+        const uint32_t cols = a.group > 1 ? static_cast<uint32_t>(a.width) : n; // of a row in this tile
+        load(first + t * kBackTile, n);
+        stage(n);
+        if constexpr (RMS) { // whole steps of four: -0 leaves a sum as it is
+            const uint32_t pad = (4 - cols % 4) % 4;
+            for (uint32_t i = tid; i < 2 * rows * pad; i += kBlock) {
+                const uint32_t c = i / pad;
+                s_rows[(c < rows ? c : a.group + c - rows) * a.ld + cols + i % pad] = -0.0f;
+            }
+        }
+        __syncthreads();
+        if constexpr (RMS) {
+            // Chain c < rows adds row c's squares, c >= rows row c - rows's
+            // products; a wave runs sixteen.
+            if (16 * wave < 2 * rows) {
+                const uint32_t c = min(16 * wave + lane % 16, 2 * rows - 1);
+                const float *s = s_rows + (c < rows ? c : a.group + c - rows) * a.ld + g4;
+                const uint32_t steps = (cols + 3) / 4;
+                auto add = [&](float v) { sums = __builtin_amdgcn_mfma_f64_4x4x4f64(static_cast<double>(v), 1.0, sums, 0, 0, 0); };
+                uint32_t k = 0;
+                if (steps >= 8) { // the next eight are read while eight are added
+                    float v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = s[4 * u];
+#pragma unroll 2
+                    for (k = 8; k + 8 <= steps; k += 8) {
+                        float w[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) w[u] = s[4 * (k + u)];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) add(v[u]);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) v[u] = w[u];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) add(v[u]);
+                }
+                for (; k < steps; ++k) add(s[4 * k]);
+            }
+        } else if (wave == 0 && lane < rows) {
+            const float *p = s_p + lane * a.ld, *q = s_q + lane * a.ld;
+            auto add = [&](float4 u, float4 v) {
+                dot = __builtin_fmaf(u.x, v.x, dot);
+                dot = __builtin_fmaf(u.y, v.y, dot);
+                dot = __builtin_fmaf(u.z, v.z, dot);
+                dot = __builtin_fmaf(u.w, v.w, dot);
+            };
+            auto p4 = [&](uint32_t i) { return *reinterpret_cast<const float4 *>(p + i); };
+            auto q4 = [&](uint32_t i) { return *reinterpret_cast<const float4 *>(q + i); };
+            uint32_t c = 0;
+            if (cols >= 16) { // the next sixteen are read while sixteen are added
+                float4 u[4], v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    u[i] = p4(4 * i);
+                    v[i] = q4(4 * i);
+                }
+#pragma unroll 2
+                for (c = 16; c + 16 <= cols; c += 16) {
+                    float4 un[4], vn[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        un[i] = p4(c + 4 * i);
+                        vn[i] = q4(c + 4 * i);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) add(u[i], v[i]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        u[i] = un[i];
+                        v[i] = vn[i];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) add(u[i], v[i]);
+            }
+            for (; c + 4 <= cols; c += 4) add(p4(c), q4(c));
+            for (; c < cols; ++c) dot = __builtin_fmaf(p[c], q[c], dot);
+        }
+        if (t + 1 < tiles) __syncthreads(); // the next tile overwrites the staged one
+    }
+    if constexpr (RMS) {
+        // result of chain 16 wave + 4 (lane / 4 % 4) + lane / 16 in each of four lanes
+        const uint32_t c = 16 * wave + 4 * (lane / 4 % 4) + g4;
+        if (lane % 4 == 0 && c < 2 * rows) s_sum[c] = sums;
+        __syncthreads();
+        if (tid < rows) s_inv[tid] = 1.0 / __builtin_sqrt(s_sum[tid] / wd + static_cast<double>(a.eps));
+    } else if (wave == 0 && lane < rows) {
+        s_sum[lane] = static_cast<double>(dot);
+    }
+    __syncthreads();
+
+    for (uint64_t t = 0; t < tiles; ++t) {
+        const uint64_t left = static_cast<uint64_t>(rows) * a.width - t * kBackTile;
+        const uint32_t n = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(left < kBackTile ? left : kBackTile));
+        const uint64_t at = first + t * kBackTile;
+        const BufRsrc yr = buffer_rsrc(a.y + at, n * 4);
+        if (tiles > 1) load(at, n);
+#pragma unroll
+        for (int j = 0; j < kBackVec; ++j) {
+            const float xe[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w}, ge[4] = {gv[j].x, gv[j].y, gv[j].z, gv[j].w};
+            float o[4];
+            uint32_t r = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (a.group > 1 && (e == 0 || !FOURS)) r = min(a.by_width.div(elem(j, e)), rows - 1);
+                if constexpr (RMS) {
+                    const double xd = static_cast<double>(xe[e]), dy = static_cast<double>(ge[e]), inv = s_inv[r];
+                    o[e] = static_cast<float>(dy * inv - xd * inv * inv * inv * s_sum[rows + r] / wd);
+                } else {
+                    o[e] = xe[e] * (ge[e] - static_cast<float>(s_sum[r]));
+                }
+            }
+            if constexpr (VEC) {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, make_float4(o[0], o[1], o[2], o[3])), yr,
+                                                       index(j) * 4, 0, 0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o[e]), yr, elem(j, e) * 4, 0, 0);
+            }
         }
     }
 }
@@ -430,6 +667,50 @@ hipError_t launch_gen_norm(const GenRowArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+// Whether ordinal k of the view is element k of its memory.
+bool dense(const GView &v)
+{
+    int64_t expect = 1;
+    for (int d = 0; d < 4; ++d) {
+        if (v.ne[d] > 1 && v.st[d] != expect) return false;
+        expect *= static_cast<int64_t>(v.ne[d]);
+    }
+    return true;
+}
+
+// Rows per workgroup: as many as a tile holds, but at least 512 workgroups
+// where there are as many rows, so that both of a CU's run.  16-byte accesses
+// where every workgroup's first element is aligned.
+template <bool RMS>
+hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
+{
+    BackArgs b{};
+    b.x = static_cast<const float *>(a.x.data);
+    b.g = static_cast<const float *>(a.g.data);
+    b.y = static_cast<float *>(a.y.data);
+    b.rows = a.rows;
+    b.width = a.width;
+    b.eps = a.eps;
+    uint64_t group = a.width >= kBackTile ? 1 : kBackTile / a.width;
+    if (group > kBackRows / (RMS ? 2 : 1)) group = kBackRows / (RMS ? 2 : 1);
+    if (group > (a.rows + 511) / 512) group = (a.rows + 511) / 512;
+    if (group >= 4 && a.width % 4 != 0) group -= group % 4;
+    b.group = static_cast<uint32_t>(group);
+    const uint32_t cols = static_cast<uint32_t>(a.width < kBackTile ? a.width : kBackTile);
+    b.ld = (cols + 63) / 64 * 64 + 4;
+    b.by_width = FastDiv(cols);
+    const uint64_t blocks = (a.rows + group - 1) / group;
+    if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
+    const bool vec = group * a.width % 4 == 0 && (a.rows * a.width) % 4 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(b.x) | reinterpret_cast<uintptr_t>(b.g) | reinterpret_cast<uintptr_t>(b.y)) & 15u) == 0;
+    const uint32_t lds = 2 * b.group * b.ld * sizeof(float);
+    const dim3 grid(static_cast<uint32_t>(blocks));
+    if (vec && a.width % 4 == 0) k_back_rows<RMS, true, true><<<grid, kBlock, lds, s>>>(b);
+    else if (vec) k_back_rows<RMS, true, false><<<grid, kBlock, lds, s>>>(b);
+    else k_back_rows<RMS, false, false><<<grid, kBlock, lds, s>>>(b);
+    return hipGetLastError();
+}
+
 // Rows narrower than a wave keep one lane per row (and the reference's
 // sequential order).
 constexpr uint64_t kNormRowMin = kWave;
@@ -453,8 +734,14 @@ hipError_t launch_generic_rows(const GenRowArgs &a, hipStream_t s)
         if (a.width >= kNormRowMin) return launch_gen_norm<true>(a, s);
         k_gen_rows<GenRow::RmsNorm><<<grid, kRowBlock, 0, s>>>(a);
         break;
-    case GenRow::SoftMaxBack: k_gen_rows<GenRow::SoftMaxBack><<<grid, kRowBlock, 0, s>>>(a); break;
-    case GenRow::RmsNormBack: k_gen_rows<GenRow::RmsNormBack><<<grid, kRowBlock, 0, s>>>(a); break;
+    case GenRow::SoftMaxBack:
+        if (dense(a.x) && dense(a.g) && dense(a.y)) return launch_back<false>(a, s);
+        k_gen_rows<GenRow::SoftMaxBack><<<grid, kRowBlock, 0, s>>>(a);
+        break;
+    case GenRow::RmsNormBack:
+        if (dense(a.x) && dense(a.g) && dense(a.y)) return launch_back<true>(a, s);
+        k_gen_rows<GenRow::RmsNormBack><<<grid, kRowBlock, 0, s>>>(a);
+        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
