@@ -61,6 +61,27 @@ __device__ __forceinline__ float4 mask4(const uint16_t *m)
                        hw_fp16_to_f32(static_cast<uint16_t>(raw.y >> 16)));
 }
 
+// The same at any 2-byte address, and 128-bit accesses at any 4-byte address:
+// rows whose width is not a multiple of four start anywhere, and global
+// memory instructions take such addresses.
+__device__ __forceinline__ float4 mask4_any(const uint16_t *m)
+{
+    typedef uint16_t h4 __attribute__((ext_vector_type(4), aligned(2)));
+    const h4 raw = *reinterpret_cast<const h4 *>(m);
+    return make_float4(hw_fp16_to_f32(raw.x), hw_fp16_to_f32(raw.y), hw_fp16_to_f32(raw.z), hw_fp16_to_f32(raw.w));
+}
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld_any(const float *p)
+{
+    const v4f_any v = *reinterpret_cast<const v4f_any *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float4 ld_any_nt(const float *p)
+{
+    const v4f_any v = __builtin_nontemporal_load(reinterpret_cast<const v4f_any *>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 // f32 products rounded, then accumulated in f64 (run_rms_norm).
 __device__ __forceinline__ double sumsq4(float4 v)
 {
@@ -362,6 +383,175 @@ __global__ __launch_bounds__(BS) void k_row_vec(RowGeo g, const float *x, float 
             const double recip = 1.0 / static_cast<double>(static_cast<float>(acc));
             for (uint32_t idx = t; idx < nv; idx += kTPR) st_nt(yr + idx, div4(yr[idx], recip));
         }
+    }
+}
+
+// ---- ragged rows: contiguous dim 0, any width of at least four, any alignment --
+// soft_max, soft_max_ext and rms_norm (+weight), by the same widths and with
+// the same arithmetic as the vectorized rows; global memory instructions take
+// 128 bits at any 4-byte address.  A row's last, partial float4 is filled up
+// with a value that leaves the reduction as it is (-inf, whose exponential is
+// 0; 0 for the squares); norm has no such value and stays with the general
+// kernel.  Lanes past the row's last whole float4 repeat it, so that no load
+// waits behind another's branch.
+template <RowOp OP, int NW, int NV, bool MASK>
+__global__ __launch_bounds__(kBlock) void k_row_ragged(RowGeo g, const float *x, float *y, const float *w, MaskGeo mg,
+                                                       float eps, float scale)
+{
+    constexpr bool kSoft = OP == RowOp::SoftMax || OP == RowOp::SoftMaxExt;
+    static_assert(kSoft || kRmsOp<OP>, "a fill value that leaves the reduction as it is");
+    constexpr uint32_t kTPR = NW * kWave;  // threads per row
+    constexpr uint32_t kRPB = kBlock / kTPR; // rows per workgroup
+    __shared__ uint64_t lds_tab[32];
+    __shared__ double lds_a[kBlock / kWave];
+    __shared__ double lds_b[kBlock / kWave];
+    ExpfConsts ec;
+    if constexpr (kSoft) {
+        if (threadIdx.x < 32) lds_tab[threadIdx.x] = kExp2Table[threadIdx.x];
+        if constexpr (NW == 1) __syncthreads(); // else the maximum's barrier orders it
+        ec = expf_consts_in_vgprs();
+    }
+    const uint32_t t = threadIdx.x % kTPR;
+    const uint32_t r = kRPB == 1 ? blockIdx.x : blockIdx.x * kRPB + __builtin_amdgcn_readfirstlane(threadIdx.x / kTPR);
+    if (r >= g.rows) return; // NW == 1 only: no barrier follows
+    uint32_t i1, i2, i3;
+    row_coords(g, r, i1, i2, i3);
+    const float *xr = x + row_base(g.x_st, i1, i2, i3);
+    float *yr = y + row_base(g.y_st, i1, i2, i3);
+    const uint16_t *mr = nullptr;
+    if constexpr (MASK) {
+        const uint64_t mrow = (static_cast<uint64_t>(mg.m3.mod(i3)) * mg.m2.d + mg.m2.mod(i2)) * mg.ne1 + i1;
+        mr = mg.p + mrow * g.ncols;
+    }
+    const uint32_t whole = g.ncols / 4, rem = g.ncols % 4, nv = whole + (rem ? 1 : 0);
+    auto ext = [&](float4 v, float4 m) {
+        if constexpr (OP == RowOp::SoftMaxExt) {
+            v = mul4(v, scale);                 // OpScale
+            if constexpr (MASK) v = add4(v, m); // OpAdd(f16 mask -> f32)
+        }
+        return v;
+    };
+    auto mask_at = [&](uint32_t idx) {
+        if constexpr (MASK) return mask4_any(mr + 4 * idx);
+        return make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    // The partial float4, number `whole`, loaded by every lane (past the end:
+    // the row's last element again).
+    float4 part;
+    {
+        const float fill = kSoft ? -__builtin_inff() : 0.0f;
+        float e[3], m[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            const uint32_t at = min(4 * whole + c, g.ncols - 1);
+            e[c] = xr[at];
+            if constexpr (MASK) m[c] = hw_fp16_to_f32(mr[at]);
+        }
+        part = ext(make_float4(e[0], e[1], e[2], 0.f), make_float4(m[0], m[1], m[2], 0.f));
+        part = make_float4(rem > 0 ? part.x : fill, rem > 1 ? part.y : fill, rem > 2 ? part.z : fill, fill);
+    }
+    auto pick = [&](bool in, float4 v) {
+        return make_float4(in ? v.x : part.x, in ? v.y : part.y, in ? v.z : part.z, in ? v.w : part.w);
+    };
+    auto at = [&](uint32_t idx) { // float4 idx < nv, cached
+        const uint32_t i = min(idx, whole - 1);
+        return pick(idx < whole, ext(ld_any(xr + 4 * i), mask_at(i)));
+    };
+    auto weight = [&](uint32_t idx) {
+        if constexpr (OP == RowOp::RmsNormMul) {
+            if (idx < whole) return ld_any(w + 4 * idx);
+            const float *p = w + 4 * idx;
+            return make_float4(rem > 0 ? p[0] : 0.f, rem > 1 ? p[1] : 0.f, rem > 2 ? p[2] : 0.f, 0.f);
+        }
+        return make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    // The lane that holds the partial float4 keeps it for the end.
+    auto put = [&](uint32_t idx, float4 o) {
+        const v4f_any v = {o.x, o.y, o.z, o.w};
+        if (idx < whole) __builtin_nontemporal_store(v, reinterpret_cast<v4f_any *>(yr + 4 * idx));
+        else part = o;
+    };
+
+    if constexpr (NV > 0) {
+        float4 v[NV];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const uint32_t i = min(t + kTPR * j, whole - 1);
+            v[j] = ext(ld_any_nt(xr + 4 * i), mask_at(i));
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[j] = pick(t + kTPR * j < whole, v[j]);
+        if constexpr (kRmsOp<OP>) {
+            double acc = 0.0;
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (t + kTPR * j < nv) acc += sumsq4(v[j]);
+            acc = row_sum<NW>(acc, lds_a);
+            const float mean = static_cast<float>(acc / static_cast<double>(g.ncols));
+            const float k = rms_scale<OP>(mean, eps);
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const uint32_t idx = t + kTPR * j;
+                if (idx < nv) {
+                    float4 o = mul4(v[j], k);
+                    if constexpr (OP == RowOp::RmsNormMul) o = mul4(o, weight(idx));
+                    put(idx, o);
+                }
+            }
+        } else {
+            float mx = -__builtin_inff();
+#pragma unroll
+            for (int j = 0; j < NV; ++j) mx = __builtin_fmaxf(mx, max4(v[j])); // repeats change no maximum
+            mx = row_max<NW>(mx, lds_a);
+            double acc = 0.0;
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                if (t + kTPR * j < nv) {
+                    v[j] = exp4(sub4(v[j], mx), lds_tab, ec);
+                    acc += sum4(v[j]);
+                }
+            }
+            acc = row_sum<NW>(acc, lds_b);
+            const double recip = 1.0 / static_cast<double>(static_cast<float>(acc));
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (t + kTPR * j < nv) put(t + kTPR * j, div4(v[j], recip));
+        }
+    } else { // wider than the registers: passes over global memory
+        if constexpr (kRmsOp<OP>) {
+            double acc = 0.0;
+            for (uint32_t idx = t; idx < nv; idx += kTPR) acc += sumsq4(at(idx));
+            acc = row_sum<NW>(acc, lds_a);
+            const float mean = static_cast<float>(acc / static_cast<double>(g.ncols));
+            const float k = rms_scale<OP>(mean, eps);
+            for (uint32_t idx = t; idx < nv; idx += kTPR) {
+                float4 o = mul4(at(idx), k);
+                if constexpr (OP == RowOp::RmsNormMul) o = mul4(o, weight(idx));
+                put(idx, o);
+            }
+        } else {
+            float mx = -__builtin_inff();
+            for (uint32_t idx = t; idx < nv; idx += kTPR) mx = __builtin_fmaxf(mx, max4(at(idx)));
+            mx = row_max<NW>(mx, lds_a);
+            double acc = 0.0;
+            for (uint32_t idx = t; idx < nv; idx += kTPR) {
+                const float4 e = exp4(sub4(at(idx), mx), lds_tab, ec);
+                const v4f_any v = {e.x, e.y, e.z, e.w};
+                if (idx < whole) *reinterpret_cast<v4f_any *>(yr + 4 * idx) = v;
+                else part = e; // this lane's own; it meets the number again below
+                acc += sum4(e);
+            }
+            acc = row_sum<NW>(acc, lds_b);
+            const double recip = 1.0 / static_cast<double>(static_cast<float>(acc));
+            for (uint32_t idx = t; idx < nv; idx += kTPR)
+                put(idx, div4(idx < whole ? ld_any(yr + 4 * idx) : part, recip));
+        }
+    }
+    if (t == whole % kTPR) {
+        float *p = yr + 4 * whole;
+        if (rem > 0) p[0] = part.x;
+        if (rem > 1) p[1] = part.y;
+        if (rem > 2) p[2] = part.z;
     }
 }
 
@@ -975,6 +1165,40 @@ void launch_vec_nv(const RowGeo &g, const RowArgs &a, const MaskGeo &mg, hipStre
     else launch_vec<OP, 4, 0, false>(g, a, mg, s);
 }
 
+template <RowOp OP, int NW, int NV>
+void launch_ragged(const RowGeo &g, const RowArgs &a, const MaskGeo &mg, hipStream_t s)
+{
+    constexpr uint32_t rows_per_block = kBlock / (NW * kWave);
+    const dim3 blocks((g.rows + rows_per_block - 1) / rows_per_block);
+    const float *x = static_cast<const float *>(a.x.data);
+    float *y = static_cast<float *>(a.y.data);
+    if constexpr (OP == RowOp::SoftMaxExt) {
+        if (mg.p) {
+            k_row_ragged<OP, NW, NV, true><<<blocks, kBlock, 0, s>>>(g, x, y, a.w, mg, a.eps, a.scale);
+            return;
+        }
+    }
+    k_row_ragged<OP, NW, NV, false><<<blocks, kBlock, 0, s>>>(g, x, y, a.w, mg, a.eps, a.scale);
+}
+
+// Ragged rows, by the same widths.  soft_max_ext, 256 rows of 3001: 7.0 us;
+// 6656 rows of 3001: 33.8 us, 4.8 TB/s.  The general kernel, a wave per row
+// that decodes every element's ordinal in three passes, took 123 us for the
+// first.
+template <RowOp OP>
+void launch_ragged_nv(const RowGeo &g, const RowArgs &a, const MaskGeo &mg, hipStream_t s)
+{
+    const uint32_t nv = (g.ncols + 3) / 4;
+    if (nv <= 1 * kWave) launch_ragged<OP, 1, 1>(g, a, mg, s);
+    else if (nv <= 2 * kWave) launch_ragged<OP, 1, 2>(g, a, mg, s);
+    else if (nv <= 4 * kWave) launch_ragged<OP, 1, 4>(g, a, mg, s);
+    else if (nv <= 2 * kBlock) launch_ragged<OP, 4, 2>(g, a, mg, s);
+    else if (nv <= 4 * kBlock) launch_ragged<OP, 4, 4>(g, a, mg, s);
+    else if (nv <= 8 * kBlock) launch_ragged<OP, 4, 8>(g, a, mg, s);
+    else if (nv <= 16 * kBlock) launch_ragged<OP, 4, 16>(g, a, mg, s);
+    else launch_ragged<OP, 4, 0>(g, a, mg, s);
+}
+
 } // namespace
 
 hipError_t launch_softmax_seq(const Operand &x, const Operand &y, hipStream_t s)
@@ -1016,7 +1240,8 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
     if (a.op == RowOp::SoftMax && !a.dense_sum) return launch_softmax_seq(a.x, a.y, s);
 
     // Vectorized rows: contiguous dim 0, 16-byte aligned row starts, and the
-    // destination row r holding the same columns as the source row r.
+    // destination row r holding the same columns as the source row r; ragged
+    // rows: the same at any width and alignment.
     auto strides4 = [](const Operand &p) {
         for (int d = 1; d < 4; ++d)
             if (p.ne[d] != 1 && p.st[d] % 4 != 0) return false;
@@ -1025,10 +1250,11 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
     const bool rows_match = same_ne(a.x, a.y) || (contiguous(a.x) && contiguous(a.y));
     const bool w_ok = a.op != RowOp::RmsNormMul || (a.w_st0 == 1 && aligned16(a.w));
     const bool mask_ok = a.op != RowOp::SoftMaxExt || a.mask == nullptr || (reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0;
-    const bool vec = ncols % 4 == 0 && a.x.st[0] == 1 && a.y.st[0] == 1 && strides4(a.x) && strides4(a.y) &&
-                     aligned16(a.x.data) && aligned16(a.y.data) && rows_match && w_ok && mask_ok &&
-                     rows < 0xffffffffull && ncols < 0xffffffffull;
-    if (vec) {
+    const bool unit = a.x.st[0] == 1 && a.y.st[0] == 1 && rows_match && rows < 0xffffffffull && ncols < 0xffffffffull;
+    const bool vec = unit && ncols % 4 == 0 && strides4(a.x) && strides4(a.y) && aligned16(a.x.data) &&
+                     aligned16(a.y.data) && w_ok && mask_ok;
+    const bool ragged = unit && !vec && ncols >= 4 && (soft || a.op == RowOp::RmsNorm || (a.op == RowOp::RmsNormMul && a.w_st0 == 1));
+    if (vec || ragged) {
         // When x and y differ in shape but are both dense, row r of each is
         // the same linear range: describe both with x's extents.
         RowGeo g{};
@@ -1057,6 +1283,15 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
             mg.ne1 = static_cast<uint32_t>(a.x.ne[1]);
             mg.m2 = FastDiv(static_cast<uint32_t>(a.mask_ne2 ? a.mask_ne2 : 1));
             mg.m3 = FastDiv(static_cast<uint32_t>(a.mask_ne3 ? a.mask_ne3 : 1));
+        }
+        if (ragged) {
+            switch (a.op) {
+            case RowOp::RmsNorm: launch_ragged_nv<RowOp::RmsNorm>(g, a, mg, s); break;
+            case RowOp::RmsNormMul: launch_ragged_nv<RowOp::RmsNormMul>(g, a, mg, s); break;
+            case RowOp::SoftMax: launch_ragged_nv<RowOp::SoftMax>(g, a, mg, s); break;
+            default: launch_ragged_nv<RowOp::SoftMaxExt>(g, a, mg, s); break;
+            }
+            return hipGetLastError();
         }
         switch (a.op) {
         case RowOp::RmsNorm: launch_vec_nv<RowOp::RmsNorm>(g, a, mg, s); break;
