@@ -15,6 +15,8 @@ from __future__ import annotations
 import ctypes
 from dataclasses import dataclass
 
+import numpy as np
+
 from .abi import CIndexView
 from .views import TensorView, TensorViewMut
 
@@ -35,7 +37,7 @@ class IndexView:
             self.ptr = data
             self.len = int(length)
             self.on_host = bool(on_host)
-        elif hasattr(data, "__array_interface__"):  # numpy
+        elif isinstance(data, np.ndarray) or hasattr(data, "__array_interface__"):  # numpy
             if data.dtype.name != "int32" or not data.flags["C_CONTIGUOUS"]:
                 raise ValueError("host indices are a C-contiguous int32 array")
             self.ptr = int(data.__array_interface__["data"][0])
