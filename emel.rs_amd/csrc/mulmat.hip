@@ -12,9 +12,9 @@
 // split along the inner dimension.
 //
 // Bound by those instructions where the outputs fill the chip (k = m = 4096,
-// n = 512: F16 297 us, 58 TFLOP/s of the 73 that a large f64 product reaches;
-// F32 164 us, 105 of 153) and by the latency of their chains where they do
-// not (n = 1: 23 us, F32 33).  A lane per output that walked both operands in
+// n = 512: F16 280 us, 61 TFLOP/s of the 73 that a large f64 product reaches;
+// F32 154 us, 111 of 153) and by the latency of their chains where they do
+// not (n = 1: 24 us, F32 25).  A lane per output that walked both operands in
 // global memory took 32.1 ms for the first.
 //
 //   k_mm_tile   a workgroup per tile of the output, operands staged in LDS
@@ -249,6 +249,8 @@ __global__ __launch_bounds__(kBlock, 2) void k_mm_tile(MmArgs a)
     const bool multiplies = SMALL ? i0 + 4 * wave < a.ni : WI * WJ == kBlock / kWave || wave < WI * WJ;
     auto multiply = [&](const unsigned char *buf) {
         if constexpr (F16) {
+            // Ahead of the other wave's staging: 5% of a whole 64x64 product.
+            __builtin_amdgcn_s_setprio(2);
             const uint32_t prow = SMALL ? 4 * wave + lane % 4 : wi * FI * 16 + c16;
             const uint32_t qrow = SMALL ? c16 : wj * FJ * 16 + c16;
             const double2 *pb = reinterpret_cast<const double2 *>(buf + prow * kPRow) + g * kPSlotG;
@@ -275,21 +277,47 @@ __global__ __launch_bounds__(kBlock, 2) void k_mm_tile(MmArgs a)
                     }
                 }
             }
+            __builtin_amdgcn_s_setprio(0);
         } else {
             const float *pf = reinterpret_cast<const float *>(buf + (wi * FI * 16 + c16) * kRow) + g;
             const float *qf = reinterpret_cast<const float *>(buf + TI * kPRow) + g * kQRow + wj * FJ * 16 + c16;
-#pragma unroll 8
-            for (int s = 0; s < BK / 4; ++s) {
-                float ep[FI], eq[FJ];
-#pragma unroll
-                for (int x = 0; x < FI; ++x) ep[x] = pf[x * 4 * kRow + s * 4];
-#pragma unroll
-                for (int z = 0; z < FJ; ++z) eq[z] = qf[s * 4 * kQRow + z * 16];
+            auto mac = [&](const float (&ep)[FI], const float (&eq)[FJ]) {
 #pragma unroll
                 for (int x = 0; x < FI; ++x)
 #pragma unroll
                     for (int z = 0; z < FJ; ++z)
                         acc[x][z] = __builtin_amdgcn_mfma_f32_16x16x4f32(ep[x], eq[z], acc[x][z], 0, 0, 0);
+            };
+            auto read = [&](float (&ep)[FI], float (&eq)[FJ], int s) {
+#pragma unroll
+                for (int x = 0; x < FI; ++x) ep[x] = pf[x * 4 * kRow + s * 4];
+#pragma unroll
+                for (int z = 0; z < FJ; ++z) eq[z] = qf[s * 4 * kQRow + z * 16];
+            };
+            if constexpr (FI * FJ == 1) {
+                // one chain: the next eight steps are read while eight are
+                // multiplied (k = m = 4096, n = 16: 25 us against 34)
+                constexpr int kStep = 8, kGroups = BK / 4 / kStep;
+                float ep[2][kStep][FI], eq[2][kStep][FJ];
+#pragma unroll
+                for (int s = 0; s < kStep; ++s) read(ep[0][s], eq[0][s], s);
+#pragma unroll
+                for (int i = 0; i < kGroups; ++i) {
+                    if (i + 1 < kGroups) {
+#pragma unroll
+                        for (int s = 0; s < kStep; ++s) read(ep[(i + 1) % 2][s], eq[(i + 1) % 2][s], (i + 1) * kStep + s);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int s = 0; s < kStep; ++s) mac(ep[i % 2][s], eq[i % 2][s]);
+                }
+            } else {
+#pragma unroll 8
+                for (int s = 0; s < BK / 4; ++s) {
+                    float ep[FI], eq[FJ];
+                    read(ep, eq, s);
+                    mac(ep, eq);
+                }
             }
         }
     };
@@ -605,13 +633,13 @@ namespace {
 
 // Which tile.  A chain of matrix instructions runs at their latency, so the
 // outputs are spread over the SIMDs before tiles grow: 16x16 up to 512 of
-// them (k = m = 4096, n = 32, F16: 39 us against 53 with 32x32 and 169 with
-// 64x64; F32 35, 39, 103) and where one dimension has at most 16 (n = 16: 27,
-// 54, 170 us), 32x32 above (n = 64: 54 us against 72 and 169), and 64x64,
-// which loads and widens least per product, where its two workgroups per CU
-// fill nine tenths of their last round (n = 512: F16 317 us against 348 with
-// 32x32 and 514 with 16x16; k = 704, m = 10533, n = 283 fill 0.81 of it and
-// take 108 against 96).
+// them (k = m = 4096, n = 32, F16: 38 us against 54 with 32x32 and 165 with
+// 64x64; F32 30, 32, 87) and where one dimension has at most 16 (n = 16: 26,
+// 54, 165 us), 32x32 above (n = 64: 54 us against 67 and 164), and 64x64,
+// which loads and widens least per product, where its tiles fill nine tenths
+// of their last round of the chip's 256 CUs (n = 512: F16 278 us against 350
+// with 32x32 and 500 with 16x16, F32 158, 205, 300; n = 256: F16 164, 170,
+// 250; but k = 704, m = 10533, n = 283 fills 0.81 and takes 102 against 97).
 template <bool F16>
 void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
 {
@@ -622,9 +650,9 @@ void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
         k_mm_any<F16><<<static_cast<uint32_t>(std::min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
         return;
     }
-    const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 512;
+    const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 256;
     if (10 * t64 >= 9 * ((t64 + round - 1) / round * round))
-        launch_tile<F16, false, 2, 2, 2, 2, F16 ? 32 : 64, 2>(a, pvec, qvec, s);
+        launch_tile<F16, false, 2, 2, 2, 2, 32, 4>(a, pvec, qvec, s);
     else if (std::min(a.ni, a.nj) > 16 && tiles(a.ni, a.nj, 16) > 512)
         launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
     else
