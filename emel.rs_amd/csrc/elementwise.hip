@@ -242,16 +242,25 @@ __device__ __forceinline__ ExpCtx stage_table(uint64_t *lds)
 // ---- dense: every operand contiguous, paired by linear index -------------
 
 // Streaming policy measured on MI355X with cold buffers: non-temporal loads
-// and stores, one float4 per thread for the copy (scale), swiglu and the
-// formulas.  The one-instruction binaries (add, sub, mul) stream 8 float4
-// per lane, each wave over 512 consecutive float4: fewer, fatter waves (mul
-// at [11008,512]: 11.85 against 12.5 us).  With 8 float4 per thread swiglu,
-// the row broadcast and a 541 MB copy were slower.
+// and stores, one float4 per thread.  Eight float4 per lane, each wave over
+// 512 consecutive float4 (fewer, fatter waves), pay for the copy, add, sub and
+// mul, and only while a launch is a few generations of waves: us with one /
+// eight, copy of 17 MB 3.8 / 4.2, 34 MB 7.1 / 6.5, 45 MB 9.2 / 8.0, 78 MB
+// 14.6 / 13.5, 112 MB 20.1 / 19.4, 128 MB 22.5 / 22.9, 256 MB 42 / 46; add and
+// mul of 12 MB 3.3 / 4.3, 50 MB 9.8 / 9.5, 75 MB 13.7 / 13.6, 101 MB
+// 17.7 / 17.8 (18.0 / 17.5 where a norm reads the sum next), 117 MB
+// 20.0 / 21.7, and one token's 48 KB 1.8 / 2.8: a lane's eight loads and
+// stores come one after the other where nothing else runs.
 template <Ew OP>
 struct Stream {
     static constexpr bool kNtLoad = true;
-    static constexpr int kVpt = OP == Ew::Add || OP == Ew::Sub || OP == Ew::Mul ? 8 : 1;
 };
+template <Ew OP>
+constexpr bool kFat = OP == Ew::Copy || OP == Ew::Add || OP == Ew::Sub || OP == Ew::Mul;
+template <Ew OP> // bytes moved
+constexpr uint64_t kFatMin = OP == Ew::Copy ? 28000000 : 45000000;
+template <Ew OP>
+constexpr uint64_t kFatMax = OP == Ew::Copy ? 116000000 : 105000000;
 
 template <Ew OP, int VPT>
 __global__ __launch_bounds__(kBlock) void k_dense(const float *a, const float *b, float *o, uint64_t nvec,
@@ -583,16 +592,25 @@ hipError_t launch_op(const EwArgs &x, hipStream_t stream)
                                                                                        Scal{x.scale, x.scale2});
             return hipGetLastError();
         }
-        constexpr int vpt = Stream<OP>::kVpt;
         const uint64_t nvec = n / 4;
-        const uint64_t per_block = static_cast<uint64_t>(kBlock) * vpt;
         const uint64_t tail = n - nvec * 4;
-        uint64_t blocks = (nvec + per_block - 1) / per_block;
-        const uint64_t tail_blocks = (tail + kBlock - 1) / kBlock;
-        if (blocks < tail_blocks) blocks = tail_blocks;
+        auto blocks_of = [&](uint64_t per_block) {
+            const uint64_t blocks = (nvec + per_block - 1) / per_block;
+            const uint64_t tail_blocks = (tail + kBlock - 1) / kBlock;
+            return blocks < tail_blocks ? tail_blocks : blocks;
+        };
+        if constexpr (kFat<OP>) {
+            const uint64_t bytes = (kBin ? 12 : 8) * n;
+            if (bytes >= kFatMin<OP> && bytes <= kFatMax<OP>) {
+                const dim3 fat(static_cast<uint32_t>(blocks_of(kBlock * 8)));
+                k_dense<OP, 8><<<fat, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});
+                return hipGetLastError();
+            }
+        }
+        const uint64_t blocks = blocks_of(kBlock);
         if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
         const dim3 grid(static_cast<uint32_t>(blocks));
-        k_dense<OP, vpt><<<grid, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});
+        k_dense<OP, 1><<<grid, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});
         return hipGetLastError();
     }
 
