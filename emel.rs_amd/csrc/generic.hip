@@ -28,6 +28,8 @@
 // Operands are addressed through their own extents and element strides, the
 // reference's coordinates_for_index/byte_offset (generic.rs:896-933), walked
 // incrementally along a row instead of re-decoded per element.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "libm_replica.hpp"
@@ -193,9 +195,11 @@ __global__ __launch_bounds__(kRowBlock) void k_gen_rows(GenRowArgs a)
 //   rms_norm_back  x*x and g*x rounded to f32 by all threads, then added by
 //                  v_mfma_f64_4x4x4 against ones: four sequential f64
 //                  additions of sixteen sums in 22 cycles (a lane that
-//                  converted and added took 16 an element).
+//                  converted and added took 16 an element).  They are staged
+//                  as doubles where the chain is what a launch waits for:
+//                  widened by the chain, each step took 30 cycles.
 // Bound by those chains for few wide rows (rms_norm_back, 512 rows of 4096:
-// 27 us, of which 13 are the chain; 2027 us with a lane per row walking global
+// 24.0 us, 26.1 with floats staged; 2027 us with a lane per row walking global
 // memory) and by memory for many (soft_max_back, 16384 rows of 512: 24 us,
 // 4.2 TB/s; 192 us).
 constexpr int kBackVec = 8;                             // float4 of x and of g per thread
@@ -207,13 +211,14 @@ struct BackArgs {
     float *y; // may be x or g
     uint64_t rows, width;
     uint32_t group; // rows per workgroup; 1 when width > kBackTile
-    uint32_t ld;    // floats per staged row
+    uint32_t ld;    // elements per staged row
     FastDiv by_width; // of the tile's element index (group > 1)
     float eps;
 };
 
-// VEC: 16-byte accesses; FOURS: a thread's four elements share a row.
-template <bool RMS, bool VEC, bool FOURS>
+// VEC: 16-byte accesses; FOURS: a thread's four elements share a row; WIDE
+// (RMS): the chains' operands are staged as doubles.
+template <bool RMS, bool VEC, bool FOURS, bool WIDE>
 __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) float s_rows[];
@@ -226,8 +231,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
     const uint64_t first = r0 * a.width;
     const double wd = static_cast<double>(a.width);
     const uint64_t tiles = a.group > 1 ? 1 : (a.width + kBackTile - 1) / kBackTile;
-    float *const s_p = s_rows;
-    float *const s_q = s_rows + a.group * a.ld;
+    using Staged = typename std::conditional<WIDE, double, float>::type;
+    using Staged4 = Staged __attribute__((ext_vector_type(4), aligned(16)));
+    Staged *const s_p = reinterpret_cast<Staged *>(s_rows);
+    Staged *const s_q = s_p + a.group * a.ld;
 
     float4 xv[kBackVec], gv[kBackVec];
     auto index = [&](int j) { return VEC ? (j * kBlock + tid) * 4 : j * kBlock * 4 + tid; };
@@ -268,8 +275,8 @@ __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
             if constexpr (FOURS) {
                 if (index(j) < n) {
                     const uint32_t o = place(index(j));
-                    *reinterpret_cast<float4 *>(s_p + o) = p;
-                    *reinterpret_cast<float4 *>(s_q + o) = q;
+                    *reinterpret_cast<Staged4 *>(s_p + o) = Staged4{p.x, p.y, p.z, p.w};
+                    *reinterpret_cast<Staged4 *>(s_q + o) = Staged4{q.x, q.y, q.z, q.w};
                 }
             } else {
                 const float pe[4] = {p.x, p.y, p.z, p.w}, qe[4] = {q.x, q.y, q.z, q.w};
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
             const uint32_t pad = (4 - cols % 4) % 4;
             for (uint32_t i = tid; i < 2 * rows * pad; i += kBlock) {
                 const uint32_t c = i / pad;
-                s_rows[(c < rows ? c : a.group + c - rows) * a.ld + cols + i % pad] = -0.0f;
+                s_p[(c < rows ? c : a.group + c - rows) * a.ld + cols + i % pad] = -0.0f;
             }
         }
         __syncthreads();
@@ -308,17 +315,17 @@ __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
             // products; a wave runs sixteen.
             if (16 * wave < 2 * rows) {
                 const uint32_t c = min(16 * wave + lane % 16, 2 * rows - 1);
-                const float *s = s_rows + (c < rows ? c : a.group + c - rows) * a.ld + g4;
+                const Staged *s = s_p + (c < rows ? c : a.group + c - rows) * a.ld + g4;
                 const uint32_t steps = (cols + 3) / 4;
-                auto add = [&](float v) { sums = __builtin_amdgcn_mfma_f64_4x4x4f64(static_cast<double>(v), 1.0, sums, 0, 0, 0); };
+                auto add = [&](Staged v) { sums = __builtin_amdgcn_mfma_f64_4x4x4f64(static_cast<double>(v), 1.0, sums, 0, 0, 0); };
                 uint32_t k = 0;
                 if (steps >= 8) { // the next eight are read while eight are added
-                    float v[8];
+                    Staged v[8];
 #pragma unroll
                     for (int u = 0; u < 8; ++u) v[u] = s[4 * u];
 #pragma unroll 2
                     for (k = 8; k + 8 <= steps; k += 8) {
-                        float w[8];
+                        Staged w[8];
 #pragma unroll
                         for (int u = 0; u < 8; ++u) w[u] = s[4 * (k + u)];
 #pragma unroll
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_back_rows(BackArgs a)
                 for (; k < steps; ++k) add(s[4 * k]);
             }
         } else if (wave == 0 && lane < rows) {
-            const float *p = s_p + lane * a.ld, *q = s_q + lane * a.ld;
+            const float *p = s_rows + lane * a.ld, *q = s_rows + (a.group + lane) * a.ld;
             auto add = [&](float4 u, float4 v) {
                 dot = __builtin_fmaf(u.x, v.x, dot);
                 dot = __builtin_fmaf(u.y, v.y, dot);
@@ -704,11 +711,28 @@ hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
     const bool vec = group * a.width % 4 == 0 && (a.rows * a.width) % 4 == 0 &&
                      ((reinterpret_cast<uintptr_t>(b.x) | reinterpret_cast<uintptr_t>(b.g) | reinterpret_cast<uintptr_t>(b.y)) & 15u) == 0;
     const uint32_t lds = 2 * b.group * b.ld * sizeof(float);
-    const dim3 grid(static_cast<uint32_t>(blocks));
-    if (vec && a.width % 4 == 0) k_back_rows<RMS, true, true><<<grid, kBlock, lds, s>>>(b);
-    else if (vec) k_back_rows<RMS, true, false><<<grid, kBlock, lds, s>>>(b);
-    else k_back_rows<RMS, false, false><<<grid, kBlock, lds, s>>>(b);
-    return hipGetLastError();
+    auto go = [&](auto wide) {
+        constexpr bool WIDE = decltype(wide)::value;
+        const uint32_t bytes = WIDE ? 2 * lds : lds;
+        const dim3 grid(static_cast<uint32_t>(blocks));
+        if (vec && a.width % 4 == 0) k_back_rows<RMS, true, true, WIDE><<<grid, kBlock, bytes, s>>>(b);
+        else if (vec) k_back_rows<RMS, true, false, WIDE><<<grid, kBlock, bytes, s>>>(b);
+        else k_back_rows<RMS, false, false, WIDE><<<grid, kBlock, bytes, s>>>(b);
+        return hipGetLastError();
+    };
+    // Staged as doubles where wide rows' chains have no other workgroup's
+    // memory traffic beside them: one round of two workgroups per CU, each
+    // with half of its 160 KB of LDS (or of one, with nearly all).  us with
+    // floats / doubles: 512 rows of 4096 26.1 / 24.0, 300 of 2304 16.3 / 15.1,
+    // 1500 of 1056 12.7 / 12.2, 16 of 512 6.35 / 6.15.  More workgroups lose
+    // the others that floats leave room for, 700 of 4224 29.5 / 42.3, 2000 of
+    // 4224 65.4 / 88.1, and short chains gain less than the staging costs,
+    // 20000 of 128 12.1 / 14.7, 70000 of 64 23.6 / 25.9.
+    if constexpr (RMS) {
+        const uint32_t room = (blocks > 256 ? 78u : 156u) * 1024;
+        if (a.width >= 512 && blocks <= 512 && 2 * lds <= room) return go(std::true_type{});
+    }
+    return go(std::false_type{});
 }
 
 // Rows narrower than a wave keep one lane per row (and the reference's

@@ -65,3 +65,13 @@ def test_soft_max_back_rows_of_ordinals(gpu, row):
     # rows are runs of ordinals, whatever the extents
     x, g = normal(6, 840), normal(7, 840)
     run(gpu, G.SOFT_MAX_BACK, x, g, [6, 10, 7, 2], i32p(row))
+
+
+# either side of what is staged as doubles: width 512, a CU's LDS for two workgroups and for one, 512 workgroups,
+# groups of rows
+@pytest.mark.parametrize("width,rows", [(508, 40), (512, 40), (4928, 257), (4932, 257), (4932, 256), (4096, 512), (2050, 1025),
+                                        (1024, 2000), (1023, 2000)])
+def test_rms_norm_back_staging(gpu, width, rows):
+    n = width * rows
+    x = np.ldexp(normal(width, n), rng(8).integers(-12, 12, n)).astype(np.float32)
+    run(gpu, G.RMS_NORM_BACK, x, normal(rows, n), [width, rows, 1, 1], f32p(1e-5))
