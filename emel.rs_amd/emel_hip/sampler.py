@@ -99,6 +99,8 @@ class Sampler:
         outs = (req.selected_token_out, req.selected_score_out)
         if not all(t.is_contiguous() and t.element_size() == 4 and t.numel() >= rows for t in outs):
             st = Status(self._lib.emel_stream_synchronize(self.stream))
+            if st != Status.OK:
+                return st, None, None
             return st, *(t.reshape(-1)[:rows].cpu().numpy() for t in outs)
         keep = getattr(self._local, "keep", None)
         if keep is None or keep[0].shape[1] < rows:
