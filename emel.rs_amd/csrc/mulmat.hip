@@ -697,17 +697,19 @@ hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
         pvec = a.p_sk == 1 && a.p_si % 4 == 0 && g.k % 4 == 0 && aligned16(a.p);
         qvec = a.q_sj == 1 && a.q_sk % 4 == 0 && nj % 4 == 0 && aligned16(a.q);
     }
-    // Extents past 32 bits run in slabs.
-    const uint64_t slab = uint64_t{1} << 30;
+    // One launch takes fewer than 2^32 work-items, 2^24 tiles: larger products
+    // run in slabs of at most 2^23 of the smallest tiles.
+    const uint64_t slab_i = std::min(ni, uint64_t{1} << 22);
+    const uint64_t slab_j = (uint64_t{1} << 23) / ((slab_i + 15) / 16) * 16;
     const uint64_t es = g.f16 ? 2 : 4;
-    for (uint64_t i = 0; i < ni; i += slab)
-        for (uint64_t j = 0; j < nj; j += slab) {
+    for (uint64_t i = 0; i < ni; i += slab_i)
+        for (uint64_t j = 0; j < nj; j += slab_j) {
             MmArgs b = a;
             b.p = static_cast<const char *>(a.p) + i * es * static_cast<uint64_t>(a.p_si);
             b.q = static_cast<const char *>(a.q) + j * es * static_cast<uint64_t>(a.q_sj);
             b.y = static_cast<float *>(g.y.data) + static_cast<int64_t>(i) * a.y_si + static_cast<int64_t>(j) * a.y_sj;
-            b.ni = static_cast<uint32_t>(ni - i < slab ? ni - i : slab);
-            b.nj = static_cast<uint32_t>(nj - j < slab ? nj - j : slab);
+            b.ni = static_cast<uint32_t>(ni - i < slab_i ? ni - i : slab_i);
+            b.nj = static_cast<uint32_t>(nj - j < slab_j ? nj - j : slab_j);
             if (g.f16) launch_mm<true>(b, pvec, qvec, s);
             else launch_mm<false>(b, pvec, qvec, s);
             const hipError_t e = hipGetLastError();

@@ -1,0 +1,37 @@
+"""Extents past what one launch can index are accepted: HIP takes fewer than 2^32 work-items in a dimension, so a kernel
+loops, or a call is launched in parts.  The operands here are larger than any memory; nothing runs."""
+import pytest
+
+import emel_hip as eh
+from launch_recorder import Recorder, view
+
+F16 = eh.DType.F16
+
+
+@pytest.fixture(scope="module")
+def rec():
+    return Recorder()
+
+
+def mul_mat(k, m, n, dtype=eh.DType.F32):
+    rhs = [n, k, 1, 1] if dtype == eh.DType.F32 else [k, n, 1, 1]
+    dst = [n, m, 1, 1] if dtype == eh.DType.F32 else [m, n, 1, 1]
+    return eh.GenericEvent(eh.GenericRequest(eh.GenericOp.MUL_MAT, view(0, [k, m, 1, 1], dtype=dtype),
+                                             view(1, rhs, dtype=dtype), None, view(2, dst, mut=True)))
+
+
+def test_the_recorder_refuses_what_hip_refuses(rec):
+    # 2^33 rows of one column, a lane each
+    with pytest.raises(RuntimeError):
+        rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp.CUMSUM, view(0, [1, 1 << 33, 1, 1]), None, None,
+                                                       view(1, [1, 1 << 33, 1, 1], mut=True))))
+
+
+@pytest.mark.parametrize("k,m,n", [(64, 1 << 30, 1), (64, (1 << 30) + 5, 64), (64, 1, 1 << 31), (64, 16, 1 << 32), (256, 1 << 17, 1 << 18)])
+@pytest.mark.parametrize("dtype", [eh.DType.F32, F16])
+def test_mul_mat_extents(rec, k, m, n, dtype):
+    got = rec.launches(mul_mat(k, m, n, dtype))
+    if all("k_mm_any" in g.name or "k_mm_rows" in g.name for g in got):
+        return  # these loop over their outputs
+    tile = {"1, 1, 1, 1": 16, "1, 1, 2, 2": 32, "2, 2, 2, 2": 64}
+    assert sum(g.grid * t * t for g in got for shape, t in tile.items() if f", {shape}, " in g.name) >= m * n
