@@ -599,15 +599,18 @@ hipError_t launch_op(const EwArgs &x, hipStream_t stream)
             const uint64_t tail_blocks = (tail + kBlock - 1) / kBlock;
             return blocks < tail_blocks ? tail_blocks : blocks;
         };
+        const uint64_t blocks = blocks_of(kBlock);
         if constexpr (kFat<OP>) {
             const uint64_t bytes = (kBin ? 12 : 8) * n;
-            if (bytes >= kFatMin<OP> && bytes <= kFatMax<OP>) {
-                const dim3 fat(static_cast<uint32_t>(blocks_of(kBlock * 8)));
+            // and where one float4 per thread needs 2^32 threads, a launch's limit
+            if ((bytes >= kFatMin<OP> && bytes <= kFatMax<OP>) || blocks > 0xffffffffull / kBlock) {
+                const uint64_t wide = blocks_of(kBlock * 8);
+                if (wide > 0x7fffffffull) return hipErrorInvalidConfiguration;
+                const dim3 fat(static_cast<uint32_t>(wide));
                 k_dense<OP, 8><<<fat, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});
                 return hipGetLastError();
             }
         }
-        const uint64_t blocks = blocks_of(kBlock);
         if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
         const dim3 grid(static_cast<uint32_t>(blocks));
         k_dense<OP, 1><<<grid, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});

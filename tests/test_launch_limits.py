@@ -35,3 +35,11 @@ def test_mul_mat_extents(rec, k, m, n, dtype):
         return  # these loop over their outputs
     tile = {"1, 1, 1, 1": 16, "1, 1, 2, 2": 32, "2, 2, 2, 2": 64}
     assert sum(g.grid * t * t for g in got for shape, t in tile.items() if f", {shape}, " in g.name) >= m * n
+
+
+@pytest.mark.parametrize("event", [eh.OpAdd, eh.OpSub, eh.OpMul])
+@pytest.mark.parametrize("n", [(1 << 34) - 1024, 1 << 34, (1 << 36) + 3])
+def test_dense_binary_extents(rec, event, n):
+    got, = rec.launches(event(view(0, [n, 1, 1, 1]), view(1, [n, 1, 1, 1]), view(2, [n, 1, 1, 1], mut=True)))
+    per_lane = 32 if ", 8>" in got.name else 4
+    assert got.grid * got.block * per_lane >= n // 4 * 4
