@@ -686,8 +686,28 @@ bool dense(const GView &v)
 }
 
 // Rows per workgroup: as many as a tile holds, but at least 512 workgroups
-// where there are as many rows, so that both of a CU's run.  16-byte accesses
-// where every workgroup's first element is aligned.
+// where there are as many rows, so that both of a CU's run.
+template <bool RMS>
+uint64_t back_group(const GenRowArgs &a)
+{
+    uint64_t group = a.width >= kBackTile ? 1 : kBackTile / a.width;
+    if (group > kBackRows / (RMS ? 2 : 1)) group = kBackRows / (RMS ? 2 : 1);
+    if (group > (a.rows + 511) / 512) group = (a.rows + 511) / 512;
+    if (group >= 4 && a.width % 4 != 0) group -= group % 4;
+    return group;
+}
+
+// Dense operands go by workgroups as long as these fit a launch's 2^32
+// work-items (rows of 16 with 32 to a workgroup: 2^29 rows, 34 GB an operand;
+// a lane per row takes 2^32).
+template <bool RMS>
+bool back_by_groups(const GenRowArgs &a)
+{
+    const uint64_t group = back_group<RMS>(a);
+    return dense(a.x) && dense(a.g) && dense(a.y) && (a.rows + group - 1) / group <= 0xffffffffull / kBlock;
+}
+
+// 16-byte accesses where every workgroup's first element is aligned.
 template <bool RMS>
 hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
 {
@@ -698,16 +718,12 @@ hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
     b.rows = a.rows;
     b.width = a.width;
     b.eps = a.eps;
-    uint64_t group = a.width >= kBackTile ? 1 : kBackTile / a.width;
-    if (group > kBackRows / (RMS ? 2 : 1)) group = kBackRows / (RMS ? 2 : 1);
-    if (group > (a.rows + 511) / 512) group = (a.rows + 511) / 512;
-    if (group >= 4 && a.width % 4 != 0) group -= group % 4;
+    const uint64_t group = back_group<RMS>(a);
     b.group = static_cast<uint32_t>(group);
     const uint32_t cols = static_cast<uint32_t>(a.width < kBackTile ? a.width : kBackTile);
     b.ld = (cols + 63) / 64 * 64 + 4;
     b.by_width = FastDiv(cols);
     const uint64_t blocks = (a.rows + group - 1) / group;
-    if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
     const bool vec = group * a.width % 4 == 0 && (a.rows * a.width) % 4 == 0 &&
                      ((reinterpret_cast<uintptr_t>(b.x) | reinterpret_cast<uintptr_t>(b.g) | reinterpret_cast<uintptr_t>(b.y)) & 15u) == 0;
     const uint32_t lds = 2 * b.group * b.ld * sizeof(float);
@@ -759,11 +775,11 @@ hipError_t launch_generic_rows(const GenRowArgs &a, hipStream_t s)
         k_gen_rows<GenRow::RmsNorm><<<grid, kRowBlock, 0, s>>>(a);
         break;
     case GenRow::SoftMaxBack:
-        if (dense(a.x) && dense(a.g) && dense(a.y)) return launch_back<false>(a, s);
+        if (back_by_groups<false>(a)) return launch_back<false>(a, s);
         k_gen_rows<GenRow::SoftMaxBack><<<grid, kRowBlock, 0, s>>>(a);
         break;
     case GenRow::RmsNormBack:
-        if (dense(a.x) && dense(a.g) && dense(a.y)) return launch_back<true>(a, s);
+        if (back_by_groups<true>(a)) return launch_back<true>(a, s);
         k_gen_rows<GenRow::RmsNormBack><<<grid, kRowBlock, 0, s>>>(a);
         break;
     default: return hipErrorInvalidValue;

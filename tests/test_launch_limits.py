@@ -43,3 +43,12 @@ def test_dense_binary_extents(rec, event, n):
     got, = rec.launches(event(view(0, [n, 1, 1, 1]), view(1, [n, 1, 1, 1]), view(2, [n, 1, 1, 1], mut=True)))
     per_lane = 32 if ", 8>" in got.name else 4
     assert got.grid * got.block * per_lane >= n // 4 * 4
+
+
+@pytest.mark.parametrize("op,width,rows", [("RMS_NORM_BACK", 64, (1 << 29) + 1), ("RMS_NORM_BACK", 16, 1 << 30), ("SOFT_MAX_BACK", 32, 1 << 30),
+                                           ("SOFT_MAX_BACK", 100, (1 << 32) - 64), ("SOFT_MAX_BACK", 128, (1 << 30) - 64)])
+def test_back_rows_extents(rec, op, width, rows):
+    params = eh.OpParams.i32(width) if op == "SOFT_MAX_BACK" else eh.OpParams.f32(1e-5)
+    ne = [width, rows, 1, 1]
+    got, = rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp[op], view(0, ne), view(1, ne), None, view(2, ne, mut=True), params)))
+    assert "k_back_rows" in got.name or got.grid * got.block >= rows  # a lane per row
