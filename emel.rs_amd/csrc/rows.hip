@@ -1181,6 +1181,8 @@ void launch_ragged(const RowGeo &g, const RowArgs &a, const MaskGeo &mg, hipStre
     k_row_ragged<OP, NW, NV, false><<<blocks, kBlock, 0, s>>>(g, x, y, a.w, mg, a.eps, a.scale);
 }
 
+constexpr uint64_t kRaggedWave = 4 * 4 * kWave; // columns of a row that one wave holds
+
 // Ragged rows, by the same widths.  soft_max_ext, 256 rows of 3001: 7.0 us;
 // 6656 rows of 3001: 33.8 us, 4.8 TB/s.  The general kernel, a wave per row
 // that decodes every element's ordinal in three passes, took 123 us for the
@@ -1191,7 +1193,7 @@ void launch_ragged_nv(const RowGeo &g, const RowArgs &a, const MaskGeo &mg, hipS
     const uint32_t nv = (g.ncols + 3) / 4;
     if (nv <= 1 * kWave) launch_ragged<OP, 1, 1>(g, a, mg, s);
     else if (nv <= 2 * kWave) launch_ragged<OP, 1, 2>(g, a, mg, s);
-    else if (nv <= 4 * kWave) launch_ragged<OP, 1, 4>(g, a, mg, s);
+    else if (g.ncols <= kRaggedWave) launch_ragged<OP, 1, 4>(g, a, mg, s);
     else if (nv <= 2 * kBlock) launch_ragged<OP, 4, 2>(g, a, mg, s);
     else if (nv <= 4 * kBlock) launch_ragged<OP, 4, 4>(g, a, mg, s);
     else if (nv <= 8 * kBlock) launch_ragged<OP, 4, 8>(g, a, mg, s);
@@ -1253,7 +1255,10 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
     const bool unit = a.x.st[0] == 1 && a.y.st[0] == 1 && rows_match && rows < 0xffffffffull && ncols < 0xffffffffull;
     const bool vec = unit && ncols % 4 == 0 && strides4(a.x) && strides4(a.y) && aligned16(a.x.data) &&
                      aligned16(a.y.data) && w_ok && mask_ok;
-    const bool ragged = unit && !vec && ncols >= 4 && (soft || a.op == RowOp::RmsNorm || (a.op == RowOp::RmsNormMul && a.w_st0 == 1));
+    // A workgroup per ragged row above kRaggedWave columns, against four rows
+    // in the general kernel: past 2^32 work-items the rows stay with that.
+    const bool launchable = ncols <= kRaggedWave || rows <= 0xffffffffull / kBlock;
+    const bool ragged = unit && !vec && ncols >= 4 && launchable && (soft || a.op == RowOp::RmsNorm || (a.op == RowOp::RmsNormMul && a.w_st0 == 1));
     if (vec || ragged) {
         // When x and y differ in shape but are both dense, row r of each is
         // the same linear range: describe both with x's extents.

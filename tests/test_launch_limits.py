@@ -52,3 +52,15 @@ def test_back_rows_extents(rec, op, width, rows):
     ne = [width, rows, 1, 1]
     got, = rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp[op], view(0, ne), view(1, ne), None, view(2, ne, mut=True), params)))
     assert "k_back_rows" in got.name or got.grid * got.block >= rows  # a lane per row
+
+
+@pytest.mark.parametrize("cols,rows", [(1027, 1 << 24), (1025, (1 << 26) - 4), (1023, (1 << 26) - 4)])
+@pytest.mark.parametrize("event", ["soft_max", "soft_max_ext", "rms_norm", "rms_norm_mul"])
+def test_ragged_rows_extents(rec, event, cols, rows):
+    ne = [cols, rows, 1, 1]
+    x, y = view(0, ne), view(1, ne, mut=True)
+    got, = rec.launches({"soft_max": lambda: eh.OpSoftMax(x, y),
+                         "soft_max_ext": lambda: eh.OpSoftMaxExt(x, None, 0.5, y),
+                         "rms_norm": lambda: eh.OpRmsNorm(x, y, 1e-5),
+                         "rms_norm_mul": lambda: eh.OpRmsNormMul(x, view(2, [cols, 1, 1, 1]), y, 1e-5)}[event]())
+    assert got.grid * (4 if cols <= 1024 or "ragged" not in got.name else 1) >= rows
