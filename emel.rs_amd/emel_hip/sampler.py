@@ -109,11 +109,16 @@ class Sampler:
             host = torch.empty((2, max(rows, 64)), dtype=torch.int32, pin_memory=True)
             keep = self._local.keep = (host.numpy(), host[0].data_ptr(), host[1].data_ptr())
         host, *ptrs = keep
+        st = Status.OK
         for t, p in zip(outs, ptrs):
-            st = Status(self._lib.emel_memcpy_dtoh(p, t.data_ptr(), 4 * rows, self.stream))
-            if st != Status.OK:
-                return st, None, None
-        st = Status(self._lib.emel_stream_synchronize(self.stream))
+            if st == Status.OK:
+                st = Status(self._lib.emel_memcpy_dtoh(p, t.data_ptr(), 4 * rows, self.stream))
+        # also after a failed copy: the one before it may still write to the buffer
+        sync = Status(self._lib.emel_stream_synchronize(self.stream))
+        if st == Status.OK:
+            st = sync
+        if st != Status.OK:
+            return st, None, None
         return st, host[0, :rows], host[1, :rows].view(np.float32)
 
     def sample_temperature_top_k(self, req: SampleTemperatureTopK):
