@@ -640,6 +640,18 @@ namespace {
 // of their last round of the chip's 256 CUs (n = 512: F16 278 us against 350
 // with 32x32 and 500 with 16x16, F32 158, 205, 300; n = 256: F16 164, 170,
 // 250; but k = 704, m = 10533, n = 283 fills 0.81 and takes 102 against 97).
+//
+// Where one dimension has at most 32, a 64x64 tile is half padding or more,
+// and its tiles fill their rounds on the other dimension alone.  There 32x32
+// is faster while both operands are read along their lines: k = 4096 and
+// m = 65536, us with 16x16 / 32x32 / 64x64, F16 n = 1 207 / 339 / 555, n = 17
+// 498 / 336 / 555, k = 4095 n = 16 501 / 421 / 643; F32 n = 4 207 / 242 / 307,
+// n = 32 382 / 238 / 302.  16x16 only for whole chunks of halves: F32's
+// swings between 0.6 and 1.3 of 64x64 with the narrow side and the length.
+// Short inner dimensions do not pay for the smaller tiles' more blocks (k = 32,
+// m = 32000, n = 4, F16: 9.0 / 6.0 / 5.2), and a transposed operand is
+// gathered, so that the larger tile uses more of each line (k = 4096,
+// m = 65536, n = 1: 682 / 614 / 379).
 template <bool F16>
 void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
 {
@@ -651,12 +663,16 @@ void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
         return;
     }
     const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 256;
-    if (10 * t64 >= 9 * ((t64 + round - 1) / round * round))
-        launch_tile<F16, false, 2, 2, 2, 2, 32, 4>(a, pvec, qvec, s);
-    else if (std::min(a.ni, a.nj) > 16 && tiles(a.ni, a.nj, 16) > 512)
-        launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
-    else
-        launch_tile<F16, F16, 1, 1, 1, 1, 128, 4>(a, pvec, qvec, s);
+    const uint32_t narrow = std::min(a.ni, a.nj);
+    const bool lines = a.p_sk == 1 && (F16 || a.q_sj == 1); // k along p, j along q (F16's q: k)
+    int edge = narrow > 16 && tiles(a.ni, a.nj, 16) > 512 ? 32 : 16;
+    if (10 * t64 >= 9 * ((t64 + round - 1) / round * round)) {
+        edge = 64;
+        if (narrow <= 32 && lines && a.k >= (F16 ? 64 : 256)) edge = F16 && narrow <= 16 && pvec && a.k >= 256 ? 16 : 32;
+    }
+    if (edge == 64) launch_tile<F16, false, 2, 2, 2, 2, 32, 4>(a, pvec, qvec, s);
+    else if (edge == 32) launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
+    else launch_tile<F16, F16, 1, 1, 1, 1, 128, 4>(a, pvec, qvec, s);
 }
 
 } // namespace

@@ -61,6 +61,19 @@ def test_mul_mat_f32_tiles(gpu, k, m, n, layout):
             Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
 
 
+# one dimension of 1 to 33 beside one long enough for whole rounds of 64x64 tiles
+@pytest.mark.parametrize("k,m,n", [(264, 14850, 16), (257, 14850, 3), (72, 16390, 17), (300, 14849, 32), (64, 1, 14850),
+                                   (260, 16391, 33), (48, 14850, 9)])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_mul_mat_narrow(gpu, k, m, n, dtype):
+    lhs, rhs = values(k + m, k * m, "wide"), values(k + n, k * n, "wide")
+    if dtype == "f16":
+        lhs, rhs = (a.astype(np.float16).view(np.uint16) for a in (lhs, rhs))
+        mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [k, n, 1, 1]), Pair(np.zeros(m * n, np.float32), [m, n, 1, 1]))
+    else:
+        mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [n, k, 1, 1]), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
+
+
 def test_mul_mat_f32_underflow_keeps_signed_zeros(gpu):
     # products that round to -0 and sums that end there: the staged blocks' padding must not turn them into +0
     k, m, n = 5, 20, 18

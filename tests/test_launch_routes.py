@@ -1,0 +1,59 @@
+"""Which kernel a call takes, where the choice was measured: nothing runs, the launches are recorded."""
+import re
+
+import pytest
+
+import emel_hip as eh
+from launch_recorder import Recorder, view
+
+F32, F16 = eh.DType.F32, eh.DType.F16
+
+
+@pytest.fixture(scope="module")
+def rec():
+    return Recorder()
+
+
+def mul_mat(rec, k, m, n, dtype=F32, layout="dense"):
+    """The kernel of one product: the tile's edge, "lane" (k_mm_any) or "rows"."""
+    lnb = rnb = None
+    if layout == "lhs_columns":
+        lnb = [4 * m, 4, 4 * k * m, 4 * k * m]
+    elif layout == "rhs_columns":
+        rnb = [4 * k, 4, 4 * k * n, 4 * k * n]
+    rhs, dst = ([n, k, 1, 1], [n, m, 1, 1]) if dtype == F32 else ([k, n, 1, 1], [m, n, 1, 1])
+    got, = rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp.MUL_MAT, view(0, [k, m, 1, 1], lnb, dtype),
+                                                          view(1, rhs, rnb, dtype), None, view(2, dst, mut=True))))
+    tile = re.search(r"k_mm_tile<\w+, \w+, \w+, \w+, (\d), (\d), (\d), (\d),", got.name)
+    if tile:
+        fi, fj, wi, wj = map(int, tile.groups())
+        assert fi * wi == fj * wj
+        return 16 * fi * wi
+    return "lane" if "k_mm_any" in got.name else "rows"
+
+
+@pytest.mark.parametrize("m", [14800, 16384, 32000, 65536, 128256, 151936])
+@pytest.mark.parametrize("n", [1, 4, 16])
+def test_mul_mat_narrow_f16_takes_small_tiles(rec, m, n):
+    assert mul_mat(rec, 4096, m, n, F16) == 16
+    assert mul_mat(rec, 4096, n, m, F16) == 16  # the narrow side first
+    assert mul_mat(rec, 4095, m, n, F16) == 32  # halves gathered one by one
+    assert mul_mat(rec, 64, m, n, F16) == 32 and mul_mat(rec, 48, m, n, F16) == 64
+
+
+@pytest.mark.parametrize("m", [16384, 32000, 151936])
+@pytest.mark.parametrize("n", [2, 16, 17, 32])
+def test_mul_mat_narrow_takes_32_wide_tiles(rec, m, n):
+    assert mul_mat(rec, 4096, m, n) == mul_mat(rec, 4096, n, m) == 32
+    if n > 16:
+        assert mul_mat(rec, 4096, m, n, F16) == 32
+    # a transposed operand is gathered: the larger tile reads whole lines of it
+    assert mul_mat(rec, 4096, m, n, layout="lhs_columns") == 64
+    assert mul_mat(rec, 4096, m, n, layout="rhs_columns") == 64
+
+
+def test_mul_mat_wide_products_keep_their_tiles(rec):
+    assert mul_mat(rec, 4096, 4096, 512, F16) == mul_mat(rec, 4096, 16384, 48) == mul_mat(rec, 4096, 4096, 256) == 64
+    assert mul_mat(rec, 704, 10533, 283, F16) == mul_mat(rec, 4096, 4096, 64) == 32
+    assert mul_mat(rec, 4096, 4096, 16) == mul_mat(rec, 4096, 4096, 1, F16) == 16
+    assert mul_mat(rec, 4096, 32000, 1) == "rows"
