@@ -18,8 +18,8 @@
 // global memory took 32.1 ms for the first.
 //
 //   k_mm_tile   a workgroup per tile of the output, operands staged in LDS
-//   k_mm_any    a lane per output, for strides that a tile's 32-bit offsets
-//               cannot span
+//   k_mm_any    a lane per output, for short inner dimensions and for strides
+//               that a tile's 32-bit offsets cannot span
 //   k_mm_rows   a lane per row of lhs for one column, rows streamed through
 //               LDS: mul_mat with n = 1 and mul_mat_argmax
 //   k_mm_argmax_walk, k_mm_argmax_final
@@ -652,16 +652,40 @@ namespace {
 // m = 32000, n = 4, F16: 9.0 / 6.0 / 5.2), and a transposed operand is
 // gathered, so that the larger tile uses more of each line (k = 4096,
 // m = 65536, n = 1: 682 / 614 / 379).
+//
+// A tile also costs its launch of blocks however short the inner dimension is,
+// so up to 32 elements a lane per output may be faster (us with lanes / with
+// the tiles above: k = 1, m = 16777216, n = 1 37 / 1530, F16 38 / 2450;
+// k = 1, m = n = 1 1.8 / 3.6; k = 4, m = 1048576, n = 4 16 / 65; k = 8,
+// m = n = 8192 281 / 104).  Both are estimated, in us, from 15000 products timed
+// at k = 1 to 4096 and 1 to 16777216 outputs: the lanes' steps one after the
+// other and their loads, dearer where neighbouring outputs' elements are k
+// apart; and each tile's share of the chip.  One row or column of outputs whose
+// lanes read contiguous elements is a stream of the matrix, which a tile reads
+// in short pieces, up to longer dimensions (m = 1048576, n = 1, lhs along m:
+// k = 64 66 / 163, 512 634 / 868; lhs along k, m = 1, n = 1048576: k = 64
+// 67 / 95, 256 322 / 300; 151936 outputs, lhs along m, k = 256 82 / 65).
+template <bool F16>
+bool lanes_are_faster(const MmArgs &a, int edge, bool pvec)
+{
+    const double k = static_cast<double>(a.k), nj = static_cast<double>(a.nj), outputs = a.ni * nj;
+    const bool stream = (a.nj == 1 && a.p_si == 1) || (a.ni == 1 && a.q_sj == 1);
+    if (stream && outputs >= (1 << 19) && a.k <= (pvec ? 128 : 512)) return true;
+    if (a.k > 32) return false;
+    double apart = 0.0; // a wave takes nj columns of 64 / nj rows: rows and columns it reads, per lane
+    if (a.p_si != 1 && nj < 64) apart += 1 / nj;
+    if (a.q_sj != 1) apart += std::min(nj, 64.0) / 64;
+    const double lanes = 1.9 + 0.11 * k + outputs * 1e-6 * (1.3 + 0.6 * k + apart * (a.k < 8 ? 0.25 : 1.6) * k);
+    // a launch, and a tile of 16x16, 32x32, 64x64: operands read in 16 bytes, or one by one
+    constexpr double cost[2][4] = {{F16 ? 2.6 : 2.9, F16 ? 0.0034 : 0.0026, F16 ? 0.0039 : 0.0029, F16 ? 0.0064 : 0.0043},
+                                   {F16 ? 4.2 : 3.8, F16 ? 0.0083 : 0.0063, F16 ? 0.0057 : 0.005, F16 ? 0.01 : 0.008}};
+    const double *c = cost[!(pvec && (F16 || a.q_sj == 1))];
+    return lanes < c[0] + c[edge == 16 ? 1 : edge == 32 ? 2 : 3] * static_cast<double>(tiles(a.ni, a.nj, edge));
+}
+
 template <bool F16>
 void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
 {
-    // the largest tile's rows and block, in bytes
-    constexpr int64_t es = F16 ? 2 : 4, span = 0x7fffffff / es;
-    if (a.p_si > span / 256 || a.p_sk > span / 256 || a.q_sj > span / 256 || a.q_sk > span / 256) {
-        const uint64_t blocks = (static_cast<uint64_t>(a.ni) * a.nj + kBlock - 1) / kBlock;
-        k_mm_any<F16><<<static_cast<uint32_t>(std::min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
-        return;
-    }
     const uint64_t t64 = tiles(a.ni, a.nj, 64), round = 256;
     const uint32_t narrow = std::min(a.ni, a.nj);
     const bool lines = a.p_sk == 1 && (F16 || a.q_sj == 1); // k along p, j along q (F16's q: k)
@@ -669,6 +693,14 @@ void launch_mm(const MmArgs &a, bool pvec, bool qvec, hipStream_t s)
     if (10 * t64 >= 9 * ((t64 + round - 1) / round * round)) {
         edge = 64;
         if (narrow <= 32 && lines && a.k >= (F16 ? 64 : 256)) edge = F16 && narrow <= 16 && pvec && a.k >= 256 ? 16 : 32;
+    }
+    // and past the spans of the tiles' 32-bit offsets: the largest tile's rows and block, in bytes
+    constexpr int64_t es = F16 ? 2 : 4, span = 0x7fffffff / es;
+    const bool far = a.p_si > span / 256 || a.p_sk > span / 256 || a.q_sj > span / 256 || a.q_sk > span / 256;
+    if (far || lanes_are_faster<F16>(a, edge, pvec)) {
+        const uint64_t blocks = (static_cast<uint64_t>(a.ni) * a.nj + kBlock - 1) / kBlock;
+        k_mm_any<F16><<<static_cast<uint32_t>(std::min(blocks, uint64_t{65536})), kBlock, 0, s>>>(a);
+        return;
     }
     if (edge == 64) launch_tile<F16, false, 2, 2, 2, 2, 32, 4>(a, pvec, qvec, s);
     else if (edge == 32) launch_tile<F16, false, 1, 1, 2, 2, 64, 2>(a, pvec, qvec, s);
@@ -715,7 +747,7 @@ hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
     }
     // One launch takes fewer than 2^32 work-items, 2^24 tiles: larger products
     // run in slabs of at most 2^23 of the smallest tiles.
-    const uint64_t slab_i = std::min(ni, uint64_t{1} << 22);
+    const uint64_t slab_i = std::min(ni, uint64_t{1} << 26);
     const uint64_t slab_j = (uint64_t{1} << 23) / ((slab_i + 15) / 16) * 16;
     const uint64_t es = g.f16 ? 2 : 4;
     for (uint64_t i = 0; i < ni; i += slab_i)

@@ -74,6 +74,22 @@ def test_mul_mat_narrow(gpu, k, m, n, dtype):
         mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [n, k, 1, 1]), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
 
 
+# products that a lane per output takes, either side of a wave's columns, and transposed
+@pytest.mark.parametrize("k,m,n", [(1, 1, 1), (1, 70, 63), (2, 300, 65), (4, 5000, 64), (7, 70001, 2), (16, 1, 70001), (32, 3, 40000)])
+@pytest.mark.parametrize("layout", ["f16", "dense", "lhs_columns", "rhs_columns"])
+def test_mul_mat_short_inner_dimension(gpu, k, m, n, layout):
+    lhs, rhs, lnb, rnb = values(k + m, k * m, "special"), values(k + n, k * n, "wide"), None, None
+    if layout == "f16":
+        lhs, rhs = (a.astype(np.float16).view(np.uint16) for a in (lhs, rhs))
+        mul_mat(gpu, Pair(lhs, [k, m, 1, 1]), Pair(rhs, [k, n, 1, 1]), Pair(np.zeros(m * n, np.float32), [m, n, 1, 1]))
+        return
+    if layout == "lhs_columns":
+        lnb = [4 * m, 4, 4 * k * m, 4 * k * m]
+    elif layout == "rhs_columns":
+        rnb = [4 * k, 4, 4 * k * n, 4 * k * n]
+    mul_mat(gpu, Pair(lhs, [k, m, 1, 1], lnb), Pair(rhs, [n, k, 1, 1], rnb), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
+
+
 def test_mul_mat_f32_underflow_keeps_signed_zeros(gpu):
     # products that round to -0 and sums that end there: the staged blocks' padding must not turn them into +0
     k, m, n = 5, 20, 18

@@ -57,3 +57,21 @@ def test_mul_mat_wide_products_keep_their_tiles(rec):
     assert mul_mat(rec, 704, 10533, 283, F16) == mul_mat(rec, 4096, 4096, 64) == 32
     assert mul_mat(rec, 4096, 4096, 16) == mul_mat(rec, 4096, 4096, 1, F16) == 16
     assert mul_mat(rec, 4096, 32000, 1) == "rows"
+
+
+@pytest.mark.parametrize("dtype", [F32, F16])
+def test_mul_mat_short_inner_dimension_takes_lanes(rec, dtype):
+    for k, m, n in [(1, 1, 1), (1, 1 << 20, 4), (1, 4, 1 << 20), (1, 1 << 24, 1), (1, 4096, 4096), (2, 1 << 20, 2), (4, 1 << 20, 3),
+                    (7, 300000, 2), (16, 1, 1 << 20)]:
+        assert mul_mat(rec, k, m, n, dtype) == "lane", (k, m, n)
+    for k, m, n in [(8, 4096, 4096), (16, 4096, 512), (32, 512, 512), (64, 64, 64), (33, 1 << 20, 2)]:
+        assert mul_mat(rec, k, m, n, dtype) != "lane", (k, m, n)
+
+
+def test_mul_mat_short_inner_dimension_of_transposed_operands(rec):
+    # neighbouring lanes read neighbouring elements
+    assert mul_mat(rec, 32, 1 << 20, 1, layout="lhs_columns") == mul_mat(rec, 512, 1 << 20, 1, layout="lhs_columns") == "lane"
+    assert mul_mat(rec, 64, 1, 1 << 20) == "lane" and mul_mat(rec, 256, 1, 1 << 20) == 32
+    assert mul_mat(rec, 256, 151936, 1, layout="lhs_columns") == 64
+    assert mul_mat(rec, 8, 1, 1 << 22, layout="rhs_columns") == "lane"
+    assert mul_mat(rec, 32, 2, 1 << 20, layout="rhs_columns") == 64  # 128 bytes apart
