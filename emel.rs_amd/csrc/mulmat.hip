@@ -23,7 +23,7 @@
 //   k_mm_rows   a lane per row of lhs for one column, rows streamed through
 //               LDS: mul_mat with n = 1 and mul_mat_argmax
 //   k_mm_argmax_walk, k_mm_argmax_final
-//               mul_mat_argmax for other layouts, and its merge
+//               mul_mat_argmax for other layouts and short rows, and its merge
 #include <algorithm>
 #include <type_traits>
 
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(kWave) void k_mm_rows(const float *__restrict__ l, 
     }
 }
 
-// Other layouts: each lane walks its own row.
+// Other layouts and short rows: each lane walks its own row.
 __global__ __launch_bounds__(kBlock) void k_mm_argmax_walk(GenMatArgs a, MmBest *partial, float *row0)
 {
     const float *l = static_cast<const float *>(a.lhs.data);
@@ -599,8 +599,11 @@ constexpr uint32_t kMmPartials = 8192; // partial results of one argmax at most
 
 bool rows_vectorisable(const GView &lhs, uint64_t k, const void *h, int64_t h_st)
 {
-    // whole aligned chunks of a row, 64 rows within a buffer's 32-bit offsets
-    return lhs.st[0] == 1 && lhs.st[1] % 4 == 0 && lhs.st[1] < (int64_t{1} << 22) && k % 4 == 0 && (k == 1 || h_st == 1) &&
+    // Whole aligned chunks of a row, 64 rows within a buffer's 32-bit offsets.
+    // Rows of four leave a tile of LDS nearly empty: m = 16777216 takes
+    // 166 us here and 107 with a lane walking each row, the argmax 153 and 74
+    // (rows of eight: 186 and 275, 174 and 294).
+    return lhs.st[0] == 1 && lhs.st[1] % 4 == 0 && lhs.st[1] < (int64_t{1} << 22) && k % 4 == 0 && k >= 8 && h_st == 1 &&
            (reinterpret_cast<uintptr_t>(lhs.data) & 15u) == 0 && (reinterpret_cast<uintptr_t>(h) & 3u) == 0;
 }
 
@@ -716,7 +719,8 @@ hipError_t launch_generic_mul_mat(const GenMatArgs &g, hipStream_t s)
     uint64_t ni, nj;
     bool pvec, qvec;
     // One column: the rows' waves need to fill the chip (k = 4096, us with rows
-    // / with tiles: m = 4096 52 / 41, 11008 62 / 50, 16384 56 / 69, 32000 91 / 198).
+    // / with tiles: m = 4096 52 / 24, 11008 93 / 39, 14000 82 / 57, 16384 57 / 61,
+    // 24000 68 / 85, 32000 93 / 109).
     if (!g.f16 && g.n == 1 && g.m >= 16384 && g.m <= 0x7fffffffull && rows_vectorisable(g.lhs, g.k, g.rhs.data, g.rhs.st[1])) {
         launch_rows_dot<false>(g, nullptr, nullptr, s);
         return hipGetLastError();
@@ -774,7 +778,12 @@ hipError_t launch_generic_mul_mat_argmax(const GenMatArgs &a, hipStream_t s)
     float *row0 = reinterpret_cast<float *>(ws);
     MmBest *partial = reinterpret_cast<MmBest *>(ws + 256);
     uint32_t n;
-    if (rows_vectorisable(a.lhs, a.k, a.rhs.data, a.rhs.st[0])) {
+    // Short rows' lanes leave fewer partial results to the merge: us by rows /
+    // by lanes for rows of 8, m = 8192 5.2 / 5.8, 24000 6.5 / 5.6, 65536
+    // 6.9 / 6.1, 262144 8.6 / 10.2; of 12, 7.1 / 6.0 at 65536; of 16, 6.6 / 6.6
+    // at 24000.
+    const bool few = a.k < 16 && a.m >= 12000 && a.m < (1 << 17);
+    if (!few && rows_vectorisable(a.lhs, a.k, a.rhs.data, a.rhs.st[0])) {
         n = launch_rows_dot<true>(a, partial, row0, s);
     } else {
         const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((a.m + kBlock - 1) / kBlock, kMmPartials / (kBlock / kWave)));

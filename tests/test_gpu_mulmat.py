@@ -121,7 +121,8 @@ def argmax(gpu, lhs, rhs):
 
 # k m: row tails and tile tails of each row count per wave (16, 32, 64 rows; tiles of 128, 64, 32 columns), more row
 # blocks than workgroups, and rows that are not whole vectors
-@pytest.mark.parametrize("k,m", [(4, 1), (132, 15), (260, 33), (512, 17), (68, 65600), (36, 131137), (8, 600001), (37, 50)])
+@pytest.mark.parametrize("k,m", [(4, 1), (132, 15), (260, 33), (512, 17), (68, 65600), (36, 131137), (8, 600001), (37, 50),
+                                 (4, 70000), (8, 11999), (12, 12001), (8, 131072)])
 @pytest.mark.parametrize("case", ["plain", "tie", "zeros", "nan", "nan_first", "all_nan"])
 def test_mul_mat_argmax_rows(gpu, k, m, case):
     w, h = values(k * m, k * m, "wide"), values(k, k, "wide")
@@ -141,7 +142,7 @@ def test_mul_mat_argmax_rows(gpu, k, m, case):
     argmax(gpu, Pair(w, [k, m, 1, 1]), Pair(h, [k, 1, 1, 1]))
 
 
-@pytest.mark.parametrize("k,m", [(4, 1), (260, 33), (132, 4097), (36, 131137)])
+@pytest.mark.parametrize("k,m", [(4, 1), (260, 33), (132, 4097), (36, 131137), (4, 16390), (8, 16385)])
 def test_mul_mat_f32_one_column(gpu, k, m):
     # rhs and dst columns apart, lhs rows padded
     lhs, rhs = values(k + m, (k + 8) * m, "special"), values(k, k, "wide")

@@ -75,3 +75,29 @@ def test_mul_mat_short_inner_dimension_of_transposed_operands(rec):
     assert mul_mat(rec, 256, 151936, 1, layout="lhs_columns") == 64
     assert mul_mat(rec, 8, 1, 1 << 22, layout="rhs_columns") == "lane"
     assert mul_mat(rec, 32, 2, 1 << 20, layout="rhs_columns") == 64  # 128 bytes apart
+
+
+def argmax(rec, k, m):
+    req = eh.GenericRequest(eh.GenericOp.MUL_MAT_ARGMAX, view(0, [k, m, 1, 1]), view(1, [k, 1, 1, 1]), None,
+                            view(2, [1, 1, 1, 1], mut=True))
+
+    class Index:  # what with_index_out asks of a tensor
+        def data_ptr(self):
+            return 3 << 43
+
+        def element_size(self):
+            return 4
+
+    req.with_index_out(Index())
+    first, last = rec.launches(eh.GenericEvent(req))
+    assert "k_mm_argmax_final" in last.name
+    return "rows" if "k_mm_rows" in first.name else "walk"
+
+
+def test_rows_of_four_are_walked(rec):
+    for m in (1, 1000, 16384, 1 << 20, 1 << 24):
+        assert argmax(rec, 4, m) == "walk" and mul_mat(rec, 4, m, 1) == "lane"
+    assert mul_mat(rec, 8, 16384, 1) == mul_mat(rec, 16, 1 << 20, 1) == "rows"
+    for k in (8, 12):
+        assert [argmax(rec, k, m) for m in (1000, 11999, 12000, 65536, 1 << 17, 1 << 20)] == ["rows", "rows", "walk", "walk", "rows", "rows"]
+    assert argmax(rec, 16, 24000) == argmax(rec, 4096, 151936) == "rows"
