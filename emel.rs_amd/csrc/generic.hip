@@ -7,11 +7,12 @@
 // gives one lane the reference's whole loop for its unit of independent
 // work, in the reference's order:
 //   k_gen_rows      one lane per row: cumsum, soft_max_back and rms_norm_back
-//                   of strided operands, and norm / rms_norm rows narrower
-//                   than a wave (soft_max uses the typed strided path's exact
-//                   sequential-sum kernel);
-//   k_back_rows     soft_max_back and rms_norm_back of dense operands: the
-//                   sums as chains in order, the rest by whole workgroups;
+//                   of strided operands or narrow rows, and norm / rms_norm
+//                   rows narrower than a wave (soft_max uses the typed strided
+//                   path's exact sequential-sum kernel);
+//   k_back_rows     soft_max_back and rms_norm_back of dense operands, wider
+//                   rows: the sums as chains in order, the rest by whole
+//                   workgroups;
 //   k_gen_norm      a workgroup per row for norm and rms_norm rows of 64 or
 //                   more columns that the typed row kernels cannot take
 //                   (those run vectorisable rows with the generic arithmetic);
@@ -697,17 +698,38 @@ uint64_t back_group(const GenRowArgs &a)
     return group;
 }
 
-// Dense operands go by workgroups as long as these fit a launch's 2^32
-// work-items (rows of 16 with 32 to a workgroup: 2^29 rows, 34 GB an operand;
-// a lane per row takes 2^32).
+template <bool RMS>
+bool back_vec(const GenRowArgs &a, uint64_t group) // every workgroup's first element is 16-byte aligned
+{
+    return group * a.width % 4 == 0 && (a.rows * a.width) % 4 == 0 &&
+           ((reinterpret_cast<uintptr_t>(a.x.data) | reinterpret_cast<uintptr_t>(a.g.data) | reinterpret_cast<uintptr_t>(a.y.data)) & 15u) == 0;
+}
+
+// Dense operands of rows wide enough for a lane's 16-byte accesses and a
+// chain's reads to pay for the staging; narrower rows are read well enough by
+// a lane each.  us with lanes / workgroups:
+//   soft_max_back  1000000 rows of 1 14 / 133, 100000 of 4 5.5 / 7.8, 10000 of
+//                  4 4.1 / 3.9, 30000 of 8 6.4 / 4.1; odd widths, where a
+//                  lane's four elements span rows: 10000 of 9 5.3 / 6.6, 100 of
+//                  9 5.2 / 4.8, 30000 of 15 7.9 / 10.0, 100000 of 15 22.7 / 19.2;
+//   rms_norm_back  1000000 of 1 16 / 401, 10000 of 4 4.9 / 6.7, 10000 of 8
+//                  6.9 / 6.8, 100000 of 8 12 / 27, 100000 of 16 27.0 / 27.5;
+//                  10000 of 15 9.0 / 9.6, 10000 of 21 11.3 / 9.7.
+// And as long as the workgroups fit a launch's 2^32 work-items (rows of 16
+// with 32 to a workgroup: 2^29 rows, 34 GB an operand; a lane per row takes
+// 2^32).
 template <bool RMS>
 bool back_by_groups(const GenRowArgs &a)
 {
     const uint64_t group = back_group<RMS>(a);
-    return dense(a.x) && dense(a.g) && dense(a.y) && (a.rows + group - 1) / group <= 0xffffffffull / kBlock;
+    if (!dense(a.x) || !dense(a.g) || !dense(a.y) || (a.rows + group - 1) / group > 0xffffffffull / kBlock) return false;
+    if (a.width >= 16) return true;
+    const bool fours = a.width % 4 == 0 && back_vec<RMS>(a, group);
+    if (RMS) return a.width >= 8 && a.rows < (fours ? 16384 : 256);
+    if (fours) return a.width > 4 || a.rows < 65536;
+    return a.width >= 8 && (a.rows < 256 || (a.width >= 12 && a.rows > 65536));
 }
 
-// 16-byte accesses where every workgroup's first element is aligned.
 template <bool RMS>
 hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
 {
@@ -724,8 +746,7 @@ hipError_t launch_back(const GenRowArgs &a, hipStream_t s)
     b.ld = (cols + 63) / 64 * 64 + 4;
     b.by_width = FastDiv(cols);
     const uint64_t blocks = (a.rows + group - 1) / group;
-    const bool vec = group * a.width % 4 == 0 && (a.rows * a.width) % 4 == 0 &&
-                     ((reinterpret_cast<uintptr_t>(b.x) | reinterpret_cast<uintptr_t>(b.g) | reinterpret_cast<uintptr_t>(b.y)) & 15u) == 0;
+    const bool vec = back_vec<RMS>(a, group);
     const uint32_t lds = 2 * b.group * b.ld * sizeof(float);
     auto go = [&](auto wide) {
         constexpr bool WIDE = decltype(wide)::value;

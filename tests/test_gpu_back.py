@@ -52,6 +52,17 @@ def test_back_rows(gpu, op, width, rows, offset):
     run(gpu, op, x, g, [width, rows, 1, 1], params, offset=offset)
 
 
+# either side of what takes a lane per row
+@pytest.mark.parametrize("op", [G.SOFT_MAX_BACK, G.RMS_NORM_BACK])
+@pytest.mark.parametrize("width,rows", [(4, 65535), (4, 65536), (7, 1000), (8, 16383), (8, 16384), (9, 255), (9, 256), (12, 16385),
+                                        (15, 65537), (16, 20000)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_narrow_back_rows(gpu, op, width, rows, offset):
+    n = width * rows
+    x = np.ldexp(normal(width, n), rng(9).integers(-12, 12, n)).astype(np.float32)
+    run(gpu, op, x, normal(rows, n), [width, rows, 1, 1], i32p(width) if op == G.SOFT_MAX_BACK else f32p(1e-5), offset=offset)
+
+
 @pytest.mark.parametrize("op", [G.SOFT_MAX_BACK, G.RMS_NORM_BACK])
 @pytest.mark.parametrize("into", ["x", "g"])
 @pytest.mark.parametrize("width", [96, 8448])

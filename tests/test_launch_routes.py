@@ -101,3 +101,26 @@ def test_rows_of_four_are_walked(rec):
     for k in (8, 12):
         assert [argmax(rec, k, m) for m in (1000, 11999, 12000, 65536, 1 << 17, 1 << 20)] == ["rows", "rows", "walk", "walk", "rows", "rows"]
     assert argmax(rec, 16, 24000) == argmax(rec, 4096, 151936) == "rows"
+
+
+def back(rec, op, width, rows, offset=0):
+    ne = [width, rows, 1, 1]
+    params = eh.OpParams.i32(width) if op == "SOFT_MAX_BACK" else eh.OpParams.f32(1e-5)
+    got, = rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp[op], view(0, ne, offset=offset), view(1, ne), None,
+                                                          view(2, ne, mut=True), params)))
+    return "groups" if "k_back_rows" in got.name else "lanes"
+
+
+@pytest.mark.parametrize("op,lanes,groups", [
+    ("SOFT_MAX_BACK", [(1, 1), (1, 10000000), (3, 1000), (7, 1), (7, 1000000), (4, 100000), (9, 300), (11, 1000000), (15, 30000)],
+     [(4, 10000), (8, 100), (8, 1000000), (9, 100), (15, 100), (15, 300000), (16, 1), (17, 1000), (512, 16384)]),
+    ("RMS_NORM_BACK", [(1, 1), (2, 10000000), (4, 1), (7, 100), (9, 300), (15, 1000000), (8, 30000), (12, 100000)],
+     [(8, 1000), (12, 10000), (9, 100), (15, 100), (16, 1), (16, 100000), (21, 100000), (4096, 512)])])
+def test_narrow_gradient_rows_take_lanes(rec, op, lanes, groups):
+    assert [(w, r) for w, r in lanes if back(rec, op, w, r) != "lanes"] == []
+    assert [(w, r) for w, r in groups if back(rec, op, w, r) != "groups"] == []
+
+
+def test_narrow_gradient_rows_off_16_bytes(rec):
+    assert back(rec, "SOFT_MAX_BACK", 8, 1000, offset=4) == "lanes"  # loaded one by one, as odd widths
+    assert back(rec, "SOFT_MAX_BACK", 16, 1000, offset=4) == "groups"
