@@ -244,23 +244,37 @@ __device__ __forceinline__ ExpCtx stage_table(uint64_t *lds)
 // Streaming policy measured on MI355X with cold buffers: non-temporal loads
 // and stores, one float4 per thread.  Eight float4 per lane, each wave over
 // 512 consecutive float4 (fewer, fatter waves), pay for the copy, add, sub and
-// mul, and only while a launch is a few generations of waves: us with one /
-// eight, copy of 17 MB 3.8 / 4.2, 34 MB 7.1 / 6.5, 45 MB 9.2 / 8.0, 78 MB
-// 14.6 / 13.5, 112 MB 20.1 / 19.4, 128 MB 22.5 / 22.9, 256 MB 42 / 46; add and
-// mul of 12 MB 3.3 / 4.3, 50 MB 9.8 / 9.5, 75 MB 13.7 / 13.6, 101 MB
-// 17.7 / 17.8 (18.0 / 17.5 where a norm reads the sum next), 117 MB
-// 20.0 / 21.7, and one token's 48 KB 1.8 / 2.8: a lane's eight loads and
-// stores come one after the other where nothing else runs.
+// mul only while a launch is a few rounds of one workgroup per CU and the last
+// round is nearly full: a lane's eight loads and stores come one after the
+// other where nothing else runs.  us with one / eight:
+//   copy  16 MB (245 workgroups) 3.9 / 4.1, 26 MB 5.9 / 6.0, 28.5 MB 6.4 / 6.2,
+//         33 MB (2.0 rounds) 7.2 / 6.5, 36 MB (2.1) 7.6 / 7.8, 50 MB (3.0)
+//         10.0 / 8.7, 51 MB 10.2 / 10.1 (in cache 7.6 / 8.2), 67 MB (4.0)
+//         12.9 / 11.5, 85 MB (5.1) 15.7 / 16.0, 100 MB (6.0) 18.1 / 17.3, 117 MB
+//         (7.0) 20.9 / 20.2, 120 MB 21.5 / 22.0, 150 MB 26.0 / 29.0;
+//   add   25 MB (1.0) 5.7 / 6.0, 40 MB 8.3 / 8.7, 46 MB (1.8) 9.4 / 9.2, 50 MB
+//         (2.0) 10.0 / 9.5, 51 MB 10.2 / 11.3, 60 MB (2.4) 11.5 / 12.4, 70 MB
+//         (2.8) 13.2 / 12.6, 75 MB (3.0) 14.0 / 13.5, 76 MB 14.0 / 15.4, 95 MB
+//         (3.8) 17.4 / 17.7, 100 MB (4.0) 18.1 / 17.8 (sub 17.9 / 18.0, mul
+//         17.7 / 18.2; in cache 15.8 / 14.8, 15.6 / 15.2, 15.4 / 15.1, and with
+//         a norm reading the sum 28.8 / 28.4), 101 MB 18.0 / 20.2, 150 MB
+//         25.8 / 26.9; mul and sub otherwise within 0.4 of these.
 template <Ew OP>
 struct Stream {
     static constexpr bool kNtLoad = true;
 };
 template <Ew OP>
 constexpr bool kFat = OP == Ew::Copy || OP == Ew::Add || OP == Ew::Sub || OP == Ew::Mul;
-template <Ew OP> // bytes moved
-constexpr uint64_t kFatMin = OP == Ew::Copy ? 28000000 : 45000000;
+
+// Whether `blocks` workgroups of eight float4 per lane do: two rounds of the
+// CUs or more, up to seven (the copy) or four, with so many hundredths of them
+// full.
 template <Ew OP>
-constexpr uint64_t kFatMax = OP == Ew::Copy ? 116000000 : 105000000;
+bool fat_pays(uint64_t blocks, uint64_t cus)
+{
+    const uint64_t rounds = (blocks + cus - 1) / cus, full = OP == Ew::Copy ? 78 : rounds < 4 ? 87 : 98;
+    return rounds >= 2 && rounds <= (OP == Ew::Copy ? 7 : 4) && 100 * blocks >= full * rounds * cus;
+}
 
 template <Ew OP, int VPT>
 __global__ __launch_bounds__(kBlock) void k_dense(const float *a, const float *b, float *o, uint64_t nvec,
@@ -601,10 +615,9 @@ hipError_t launch_op(const EwArgs &x, hipStream_t stream)
         };
         const uint64_t blocks = blocks_of(kBlock);
         if constexpr (kFat<OP>) {
-            const uint64_t bytes = (kBin ? 12 : 8) * n;
+            const uint64_t wide = blocks_of(kBlock * 8);
             // and where one float4 per thread needs 2^32 threads, a launch's limit
-            if ((bytes >= kFatMin<OP> && bytes <= kFatMax<OP>) || blocks > 0xffffffffull / kBlock) {
-                const uint64_t wide = blocks_of(kBlock * 8);
+            if (fat_pays<OP>(wide, static_cast<uint64_t>(dev.cus)) || blocks > 0xffffffffull / kBlock) {
                 if (wide > 0x7fffffffull) return hipErrorInvalidConfiguration;
                 const dim3 fat(static_cast<uint32_t>(wide));
                 k_dense<OP, 8><<<fat, kBlock, 0, stream>>>(a, b, o, nvec, n, Scal{x.scale, x.scale2});

@@ -124,3 +124,21 @@ def test_narrow_gradient_rows_take_lanes(rec, op, lanes, groups):
 def test_narrow_gradient_rows_off_16_bytes(rec):
     assert back(rec, "SOFT_MAX_BACK", 8, 1000, offset=4) == "lanes"  # loaded one by one, as odd widths
     assert back(rec, "SOFT_MAX_BACK", 16, 1000, offset=4) == "groups"
+
+
+def eights(rec, op, mb):
+    """Whether the dense copy or binary that moves `mb` MB takes eight float4 per lane."""
+    n = int(mb * 1e6 / (8 if op == "copy" else 12)) // 4 * 4
+    a, b, y = view(0, [n, 1, 1, 1]), view(1, [n, 1, 1, 1]), view(2, [n, 1, 1, 1], mut=True)
+    got, = rec.launches({"copy": lambda: eh.DenseOpDup(a.ptr, y.ptr, n, n), "add": lambda: eh.OpAdd(a, b, y), "sub": lambda: eh.OpSub(a, b, y),
+                         "mul": lambda: eh.OpMul(a, b, y)}[op]())
+    return ", 8>" in got.name
+
+
+@pytest.mark.parametrize("op,few,many", [
+    ("copy", [1, 16, 20, 26, 34, 36, 51, 120, 150], [28.5, 33, 40, 50, 60, 67, 70, 80, 95, 110, 117]),
+    ("add", [1, 12, 25, 26, 40, 51, 60, 76, 83, 90, 95, 101, 104, 115, 125, 200], [46, 50, 67.6, 70, 75, 100]),
+    ("sub", [55, 80, 101], [46, 50, 75]), ("mul", [55, 80, 101], [46, 50, 75])])
+def test_dense_streams_take_eights_where_their_last_round_is_full(rec, op, few, many):
+    assert [mb for mb in few if eights(rec, op, mb)] == []
+    assert [mb for mb in many if not eights(rec, op, mb)] == []
