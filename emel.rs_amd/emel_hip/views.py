@@ -36,7 +36,8 @@ class Layout:
 
     def wire(self) -> bytes:
         """The C view of this layout without its data: a call copies it and
-        fills the pointer and size in (0.2 us, against 0.7 field by field)."""
+        fills the pointer and size in (0.2 us, against 0.7 field by field,
+        which a layout's first call pays too)."""
         if self._wire is None:
             v = CView()
             v.dtype = self.dtype
