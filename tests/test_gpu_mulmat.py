@@ -31,8 +31,8 @@ def values(seed, n, kind):
     return x
 
 
-# k m n: one element, tile and block edges of each tile (16, 32, 64 outputs; blocks of 64 to 512), k and n that are
-# not whole vectors, and outputs enough for the largest tiles
+# k m n: one element, edges of the tiles (16 and 32 outputs, and one whole number of 64s) and of one or two of their
+# blocks, k and n that are not whole vectors; longer inner dimensions in test_mul_mat_deep_tiles
 SHAPES = [(1, 1, 1), (8, 16, 16), (520, 17, 16), (511, 15, 300), (96, 4096, 1), (1032, 40, 4), (264, 33, 65),
           (260, 33, 64), (128, 100, 31), (72, 2049, 1025), (67, 2050, 1023), (64, 2048, 1024)]
 
@@ -88,6 +88,66 @@ def test_mul_mat_short_inner_dimension(gpu, k, m, n, layout):
     elif layout == "rhs_columns":
         rnb = [4 * k, 4, 4 * k * n, 4 * k * n]
     mul_mat(gpu, Pair(lhs, [k, m, 1, 1], lnb), Pair(rhs, [n, k, 1, 1], rnb), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
+
+
+# Each tile's loop over blocks at work: the 64x64 tile's (blocks of 32, four in flight) from 161 inner elements, with
+# every remainder of its four, whole vectors or not; 32x32 (blocks of 64, two) from 193; 16x16 (128, four) from 641.
+# Rows and columns end inside a tile.
+DEEP = [(64, 161, 1001, 963), (64, 200, 1001, 964), (64, 256, 1000, 964), (64, 260, 1001, 963), (64, 328, 1001, 964), (64, 385, 1001, 963),
+        (32, 200, 1000, 300), (32, 301, 1000, 300), (32, 464, 999, 301), (16, 648, 33, 17), (16, 1501, 20, 5), (16, 1536, 50, 30)]
+
+
+def deep_operands(k, m, n, layout):
+    """(lhs [m, k], rhs [k, n]) as matrices, and the operands that hold them."""
+    a, b = values(k + m, m * k, "wide").reshape(m, k), values(k + n, k * n, "wide").reshape(k, n)
+    if layout == "f16":
+        a, b = a.astype(np.float16), b.astype(np.float16)
+        return a, b, Pair(a.reshape(-1).view(np.uint16), [k, m, 1, 1]), Pair(np.ascontiguousarray(b.T).reshape(-1).view(np.uint16), [k, n, 1, 1])
+    lnb = rnb = None
+    left, right = a, b
+    if layout == "lhs_columns":
+        left, lnb = np.ascontiguousarray(a.T), [4 * m, 4, 4 * k * m, 4 * k * m]
+    elif layout == "rhs_columns":
+        right, rnb = np.ascontiguousarray(b.T), [4 * k, 4, 4 * k * n, 4 * k * n]
+    elif layout == "padded":
+        left, lnb = np.pad(a, ((0, 0), (0, 3))), [4, 4 * (k + 3)] + [4 * (k + 3) * m] * 2
+        right, rnb = np.pad(b, ((0, 0), (0, 5))), [4, 4 * (n + 5)] + [4 * (n + 5) * k] * 2
+    return a, b, Pair(left.reshape(-1), [k, m, 1, 1], lnb), Pair(right.reshape(-1), [n, k, 1, 1], rnb)
+
+
+@pytest.mark.parametrize("layout", ["f16", "dense", "lhs_columns", "rhs_columns", "padded"])
+@pytest.mark.parametrize("tile,k,m,n", DEEP)
+def test_mul_mat_deep_tiles(gpu, tile, k, m, n, layout):
+    # The oracle's loop over all outputs takes ten seconds: it checks the bits of rows at the tiles' edges, every
+    # column, and of columns at the edges, every row; 64 bits the rest.
+    a, b, lhs, rhs = deep_operands(k, m, n, layout)
+    f16 = layout == "f16"
+    dst = Pair(np.full(m * n, 7.0, np.float32), [m, n, 1, 1] if f16 else [n, m, 1, 1]).to(gpu)
+    req = eh.GenericRequest(eh.GenericOp.MUL_MAT, lhs.to(gpu).pview(), rhs.to(gpu).pview(), None, dst.pview(True))
+    assert eh.Kernel().process_event(eh.GenericEvent(req)) == eh.Status.OK, eh.last_error()
+    got = dst.result().reshape(n, m).T if f16 else dst.result().reshape(m, n)
+
+    def oracle(rows, cols):
+        x, z = a[rows], np.ascontiguousarray(b[:, cols])
+        want = np.zeros(len(rows) * len(cols), np.float32)
+        if f16:
+            views = (orc.view(x.view(np.uint16).reshape(-1), [k, len(rows), 1, 1], None, orc.F16),
+                     orc.view(np.ascontiguousarray(z.T).view(np.uint16).reshape(-1), [k, len(cols), 1, 1], None, orc.F16))
+        else:
+            views = orc.view(x.reshape(-1), [k, len(rows), 1, 1]), orc.view(z.reshape(-1), [len(cols), k, 1, 1])
+        ne = [len(rows), len(cols), 1, 1] if f16 else [len(cols), len(rows), 1, 1]
+        assert orc.generic(eh.GenericOp.MUL_MAT, *views, None, orc.view(want, ne), b"", 0, 0, None) == orc.OK
+        return want.reshape(len(cols), len(rows)).T if f16 else want.reshape(len(rows), len(cols))
+
+    edges = lambda d: sorted({i for i in (0, 1, 15, 16, 31, 32, 47, 63, 64, 65, d // 2, d - 2, d - 1) if i < d})  # noqa: E731
+    rows, cols = edges(m), edges(n)
+    what = f"{layout} {tile} k{k}"
+    assert_bits_equal(got[rows], oracle(rows, list(range(n))), what + " rows")
+    assert_bits_equal(np.ascontiguousarray(got[:, cols]), oracle(list(range(m)), cols), what + " columns")
+    exact, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    # k roundings of the sum in 32 bits (F32), or in 64 with those of `exact` itself (F16), and the result's to 32
+    bound = (2 * k * 2.0**-53 if f16 else k * 2.0**-24) * size + 2.0**-24 * np.abs(exact)
+    assert (np.abs(got - exact) <= bound).all(), what
 
 
 def test_mul_mat_f32_underflow_keeps_signed_zeros(gpu):

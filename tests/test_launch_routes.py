@@ -142,3 +142,17 @@ def eights(rec, op, mb):
 def test_dense_streams_take_eights_where_their_last_round_is_full(rec, op, few, many):
     assert [mb for mb in few if eights(rec, op, mb)] == []
     assert [mb for mb in many if not eights(rec, op, mb)] == []
+
+
+def test_the_deep_products_reach_their_tiles(rec):
+    from test_gpu_mulmat import DEEP
+
+    blocks = {16: (128, 4), 32: (64, 2), 64: (32, 4)}  # elements per block, blocks in flight
+    for tile, k, m, n in DEEP:
+        size, flight = blocks[tile]
+        assert -(-k // size) > flight + 1, (tile, k)  # the loop over blocks runs
+        for dtype in (F32, F16):
+            assert mul_mat(rec, k, m, n, dtype) == tile, (tile, k, m, n)
+        for layout in ("lhs_columns", "rhs_columns"):
+            assert mul_mat(rec, k, m, n, layout=layout) == tile
+    assert {-(-k // 32) % 4 for tile, k, _, _ in DEEP if tile == 64} == {0, 1, 2, 3}
