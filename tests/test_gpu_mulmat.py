@@ -168,6 +168,21 @@ def test_mul_mat_f32_rows_far_apart(gpu):
             Pair(values(2, k * n, "wide"), [n, k, 1, 1]), Pair(np.zeros(m * n, np.float32), [n, m, 1, 1]))
 
 
+@pytest.mark.parametrize("m,n", [((1 << 26) + 77, 1), (1, (1 << 27) + 77), (3, (1 << 27) + 5)])
+def test_mul_mat_more_outputs_than_one_launch(gpu, m, n):
+    # k = 1: every output is one product, rounded, plus +0
+    import torch
+
+    g = torch.Generator(device=gpu).manual_seed(m)
+    a, b = torch.randn(m, device=gpu, generator=g), torch.randn(n, device=gpu, generator=g)
+    y = torch.full((m * n,), 7.0, device=gpu)
+    dense = lambda t, ne, cls=eh.TensorView: cls(t, eh.Layout.dense(eh.DType.F32, ne))  # noqa: E731
+    req = eh.GenericRequest(eh.GenericOp.MUL_MAT, dense(a, [1, m, 1, 1]), dense(b, [n, 1, 1, 1]), None,
+                            dense(y, [n, m, 1, 1], eh.TensorViewMut))
+    assert eh.Kernel().process_event(eh.GenericEvent(req)) == eh.Status.OK, eh.last_error()
+    assert torch.equal(y.view(m, n), a[:, None] * b[None, :])
+
+
 def argmax(gpu, lhs, rhs):
     dst, idx = Pair(np.zeros(1, np.float32), [1, 1, 1, 1]).to(gpu), np.full(1, -7, np.int32)
     want = orc.generic(eh.GenericOp.MUL_MAT_ARGMAX, lhs.oview(), rhs.oview(), None, dst.oview(), b"", 0, 0, idx)

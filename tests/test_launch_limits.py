@@ -64,3 +64,8 @@ def test_ragged_rows_extents(rec, event, cols, rows):
                          "rms_norm": lambda: eh.OpRmsNorm(x, y, 1e-5),
                          "rms_norm_mul": lambda: eh.OpRmsNormMul(x, view(2, [cols, 1, 1, 1]), y, 1e-5)}[event]())
     assert got.grid * (4 if cols <= 1024 or "ragged" not in got.name else 1) >= rows
+
+
+def test_products_of_2_to_the_27_outputs_take_two_launches(rec):
+    for m, n in (((1 << 26) + 77, 1), (1, (1 << 27) + 77), (3, (1 << 27) + 5)):
+        assert len(rec.launches(mul_mat(1, m, n))) == 2
