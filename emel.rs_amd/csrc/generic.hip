@@ -687,14 +687,21 @@ bool dense(const GView &v)
 }
 
 // Rows per workgroup: as many as a tile holds, but at least 512 workgroups
-// where there are as many rows, so that both of a CU's run.
+// where there are as many rows, so that both of a CU's run; of odd widths a
+// multiple of four, for 16-byte accesses (more rather than fewer, which would
+// leave a few workgroups to a second round: 30001 rows of 17, soft_max_back
+// 10.2 us by 56, 7.2 by 60).
 template <bool RMS>
 uint64_t back_group(const GenRowArgs &a)
 {
-    uint64_t group = a.width >= kBackTile ? 1 : kBackTile / a.width;
-    if (group > kBackRows / (RMS ? 2 : 1)) group = kBackRows / (RMS ? 2 : 1);
-    if (group > (a.rows + 511) / 512) group = (a.rows + 511) / 512;
-    if (group >= 4 && a.width % 4 != 0) group -= group % 4;
+    uint64_t most = a.width >= kBackTile ? 1 : kBackTile / a.width;
+    if (most > kBackRows / (RMS ? 2 : 1)) most = kBackRows / (RMS ? 2 : 1);
+    uint64_t group = (a.rows + 511) / 512;
+    if (group > most) group = most;
+    if (group >= 4 && a.width % 4 != 0) {
+        group = (group + 3) / 4 * 4;
+        if (group > most) group -= 4;
+    }
     return group;
 }
 
@@ -708,13 +715,16 @@ bool back_vec(const GenRowArgs &a, uint64_t group) // every workgroup's first el
 // Dense operands of rows wide enough for a lane's 16-byte accesses and a
 // chain's reads to pay for the staging; narrower rows are read well enough by
 // a lane each.  us with lanes / workgroups:
-//   soft_max_back  1000000 rows of 1 14 / 133, 100000 of 4 5.5 / 7.8, 10000 of
-//                  4 4.1 / 3.9, 30000 of 8 6.4 / 4.1; odd widths, where a
-//                  lane's four elements span rows: 10000 of 9 5.3 / 6.6, 100 of
-//                  9 5.2 / 4.8, 30000 of 15 7.9 / 10.0, 100000 of 15 22.7 / 19.2;
+//   soft_max_back  1000000 rows of 1 14 / 133, 60000 of 4 4.9 / 5.7, 10000 of
+//                  4 4.1 / 3.9, 30000 of 8 6.4 / 4.1; odd widths and starts off
+//                  16 bytes, where a lane's four elements span rows or are
+//                  loaded one by one: 10000 of 9 5.3 / 6.6, 300 of 13 6.2 / 5.9,
+//                  100000 of 13 15.7 / 19.5, 300001 of 13 72 / 48, 20000 of 15
+//                  7.6 / 7.2;
 //   rms_norm_back  1000000 of 1 16 / 401, 10000 of 4 4.9 / 6.7, 10000 of 8
-//                  6.9 / 6.8, 100000 of 8 12 / 27, 100000 of 16 27.0 / 27.5;
-//                  10000 of 15 9.0 / 9.6, 10000 of 21 11.3 / 9.7.
+//                  6.9 / 6.8, 100000 of 8 12 / 27, 100000 of 16 27.0 / 27.5; odd
+//                  ones 10000 of 15 9.0 / 9.6, 10000 of 17 9.8 / 9.3, 60000 of 17
+//                  15.6 / 30, 60000 of 23 26 / 30, 300001 of 17 169 / 132.
 // And as long as the workgroups fit a launch's 2^32 work-items (rows of 16
 // with 32 to a workgroup: 2^29 rows, 34 GB an operand; a lane per row takes
 // 2^32).
@@ -723,11 +733,15 @@ bool back_by_groups(const GenRowArgs &a)
 {
     const uint64_t group = back_group<RMS>(a);
     if (!dense(a.x) || !dense(a.g) || !dense(a.y) || (a.rows + group - 1) / group > 0xffffffffull / kBlock) return false;
-    if (a.width >= 16) return true;
+    if (a.width >= 24) return true;
     const bool fours = a.width % 4 == 0 && back_vec<RMS>(a, group);
-    if (RMS) return a.width >= 8 && a.rows < (fours ? 16384 : 256);
-    if (fours) return a.width > 4 || a.rows < 65536;
-    return a.width >= 8 && (a.rows < 256 || (a.width >= 12 && a.rows > 65536));
+    if (RMS) {
+        if (fours) return a.width >= 16 || (a.width >= 8 && a.rows < 16384);
+        if (a.width >= 16) return a.rows < 16384 || a.rows >= 131072;
+        return a.width >= 8 && a.rows < 256;
+    }
+    if (fours) return a.width > 4 || a.rows < 32768;
+    return a.width >= 14 || (a.width >= 8 && (a.rows < 512 || (a.width >= 11 && a.rows * a.width >= (1 << 21))));
 }
 
 template <bool RMS>

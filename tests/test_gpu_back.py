@@ -54,8 +54,9 @@ def test_back_rows(gpu, op, width, rows, offset):
 
 # either side of what takes a lane per row
 @pytest.mark.parametrize("op", [G.SOFT_MAX_BACK, G.RMS_NORM_BACK])
-@pytest.mark.parametrize("width,rows", [(4, 65535), (4, 65536), (7, 1000), (8, 16383), (8, 16384), (9, 255), (9, 256), (12, 16385),
-                                        (15, 65537), (16, 20000)])
+@pytest.mark.parametrize("width,rows", [(4, 32767), (4, 32768), (7, 1000), (8, 16383), (8, 16384), (9, 255), (9, 512), (12, 16385),
+                                        (11, 190650), (11, 190651), (13, 511), (13, 512), (14, 600), (15, 65537), (16, 20000),
+                                        (17, 4097), (17, 16384), (18, 30001), (23, 131072)])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_narrow_back_rows(gpu, op, width, rows, offset):
     n = width * rows

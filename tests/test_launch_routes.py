@@ -112,18 +112,27 @@ def back(rec, op, width, rows, offset=0):
 
 
 @pytest.mark.parametrize("op,lanes,groups", [
-    ("SOFT_MAX_BACK", [(1, 1), (1, 10000000), (3, 1000), (7, 1), (7, 1000000), (4, 100000), (9, 300), (11, 1000000), (15, 30000)],
-     [(4, 10000), (8, 100), (8, 1000000), (9, 100), (15, 100), (15, 300000), (16, 1), (17, 1000), (512, 16384)]),
-    ("RMS_NORM_BACK", [(1, 1), (2, 10000000), (4, 1), (7, 100), (9, 300), (15, 1000000), (8, 30000), (12, 100000)],
-     [(8, 1000), (12, 10000), (9, 100), (15, 100), (16, 1), (16, 100000), (21, 100000), (4096, 512)])])
+    ("SOFT_MAX_BACK", [(1, 1), (1, 10000000), (3, 1000), (7, 1), (7, 1000000), (4, 60000), (9, 512), (10, 1000000), (13, 100000)],
+     [(4, 30000), (8, 100), (8, 1000000), (9, 300), (13, 300), (13, 300000), (11, 1000000), (14, 1), (15, 30000), (17, 1000), (512, 16384)]),
+    ("RMS_NORM_BACK", [(1, 1), (2, 10000000), (4, 1), (7, 100), (9, 300), (15, 1000000), (8, 30000), (12, 100000), (17, 60000), (23, 100000)],
+     [(8, 1000), (12, 10000), (9, 100), (15, 100), (16, 1), (16, 100000), (17, 10000), (17, 300000), (24, 60000), (4096, 512)])])
 def test_narrow_gradient_rows_take_lanes(rec, op, lanes, groups):
     assert [(w, r) for w, r in lanes if back(rec, op, w, r) != "lanes"] == []
     assert [(w, r) for w, r in groups if back(rec, op, w, r) != "groups"] == []
 
 
 def test_narrow_gradient_rows_off_16_bytes(rec):
-    assert back(rec, "SOFT_MAX_BACK", 8, 1000, offset=4) == "lanes"  # loaded one by one, as odd widths
-    assert back(rec, "SOFT_MAX_BACK", 16, 1000, offset=4) == "groups"
+    # loaded one by one, as odd widths
+    assert back(rec, "SOFT_MAX_BACK", 8, 1000, offset=4) == back(rec, "RMS_NORM_BACK", 16, 60000, offset=4) == "lanes"
+    assert back(rec, "SOFT_MAX_BACK", 16, 1000, offset=4) == back(rec, "RMS_NORM_BACK", 24, 60000, offset=4) == "groups"
+
+
+@pytest.mark.parametrize("width,rows", [(17, 4097), (18, 30001), (1023, 2500), (513, 3100)])
+def test_gradient_rows_of_odd_widths_run_in_one_round(rec, width, rows):
+    ne = [width, rows, 1, 1]
+    got, = rec.launches(eh.GenericEvent(eh.GenericRequest(eh.GenericOp.SOFT_MAX_BACK, view(0, ne), view(1, ne), None,
+                                                          view(2, ne, mut=True), eh.OpParams.i32(width))))
+    assert "k_back_rows" in got.name and got.grid <= 512  # two workgroups on each of 256 CUs
 
 
 def eights(rec, op, mb):
